@@ -21,6 +21,8 @@
 //    one subject query against tens of comparables).  HBM-bound: each wave
 //    owns one query row, streams the plane's K and V once with coalesced
 //    128-bit loads straight into registers and reduces with DPP.
+//  * rbf_split_kernel   -- the same for more than one key tile: the waves of a
+//    workgroup share a row's key axis.
 //  * rbf_generic_kernel -- any strides, head dims and alignments.
 //  * rbf_mfma_kernel (rbf_mfma.hip) -- query tiles on bf16/fp16 MFMA.
 
@@ -39,16 +41,14 @@ namespace vectra {
 // chunk of exactly the keys whose weights it computed and P.V needs no
 // shuffle until the final reduction.
 //
-// Scheduling: the grid is persistent (a fixed number of waves, each taking
-// query rows wave, wave + waves, ...).  A wave always has its next work item
-// (a row and 64-key tile) in flight while it reduces the current one, so the
-// softmax and P.V arithmetic of one row overlaps the HBM stream of the next;
-// a one-shot grid instead leaves every wave waiting for its last bytes until
-// the end of the stream and then serialises all of its arithmetic.  Every
-// load of a work item (K, V, the key bias, and at a row's first tile q and
-// the coefficient) is issued together; rows past Nk are loaded from row
-// Nk - 1 (always in bounds) and masked afterwards, so no load is behind a
-// branch.  Per-lane addresses are 32-bit offsets from wave-uniform bases.
+// Scheduling: one key tile per row (Nk <= 64; longer key axes take the split
+// kernel below).  Where a wave takes several rows, it has the next one in
+// flight while it reduces the current one, so the softmax and P.V arithmetic
+// of one row overlaps the HBM stream of the next.  Every load of a row (K, V,
+// the key bias, q and the coefficient) is issued together; rows past Nk are
+// loaded from row Nk - 1 (always in bounds) and masked afterwards, so no load
+// is behind a branch.  Per-lane addresses are 32-bit offsets from
+// wave-uniform bases.
 // ------------------------------------------------------------------------
 
 // Sums kVec accumulators per lane over the row-group lane bits (kChunks ..
@@ -119,13 +119,11 @@ __device__ __forceinline__ RowCoords row_coords(int32_t row, const Problem& p) {
 template <typename T, typename OutT, int kChunks, int kRows>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 void rbf_stream_kernel(Problem p) {
-  // kRows > 0: the wave takes rows wave * kRows .. + kRows - 1, each one key
-  // tile (Nk <= 64), in a fully unrolled pipeline with no loop and no branch
+  // The wave takes rows wave * kRows .. + kRows - 1, each one key tile
+  // (Nk <= 64), in a fully unrolled pipeline with no loop and no branch
   // around a load, so the compiler can wait for exactly the loads each step
   // needs.  Rows past the end are clamped to the last row: the duplicate
   // wave recomputes that row and stores the same bytes.
-  // kRows == 0: rows wave, wave + grid_waves, ..., any number of key tiles.
-  constexpr bool kSingleTile = kRows > 0;
   constexpr int kVec = Vec<T>::kN;
   constexpr int kRowsPerPass = kWave / kChunks;
   constexpr int kPasses = kChunks;  // kPasses * kRowsPerPass == 64 keys
@@ -142,7 +140,7 @@ void rbf_stream_kernel(Problem p) {
       static_cast<int32_t>(blockIdx.x) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int32_t total_rows = static_cast<int32_t>(p.total_rows);
   // No barriers below: early exit is safe.
-  if (wave_id * (kRows > 0 ? kRows : 1) >= total_rows) return;
+  if (wave_id * kRows >= total_rows) return;
 
   const int32_t n_waves = p.grid_waves;
   const int32_t n_k = static_cast<int32_t>(p.Nk);
@@ -167,45 +165,36 @@ void rbf_stream_kernel(Problem p) {
     }
     return;
   }
-  const int32_t tiles = kSingleTile ? 1 : (n_k + kWave - 1) / kWave;
 
-  // Per-lane byte offsets of a tile's keys inside a (b, h) plane.  Those of
-  // tile 0 are the same for every row, so they are computed once: issuing
-  // the next row's loads then only changes wave-uniform base addresses.
+  // Per-lane byte offsets of the keys inside a (b, h) plane.  They are the
+  // same for every row, so they are computed once: issuing the next row's
+  // loads then only changes wave-uniform base addresses.
   struct Offsets {
     uint32_t k[kPasses], v[kPasses], bias[kPasses];
   };
-  auto tile_offsets = [&](int32_t tile) {
-    Offsets o;
+  Offsets o;
 #pragma unroll
-    for (int s = 0; s < kPasses; ++s) {
-      const int32_t j = tile * kWave + s * kRowsPerPass + group;
-      const uint32_t key = static_cast<uint32_t>(j < n_k - 1 ? j : n_k - 1);
-      o.k[s] = key * k_row_bytes + chunk_bytes;
-      o.v[s] = key * v_row_bytes + chunk_bytes;
-      o.bias[s] = key * static_cast<uint32_t>(p.sbn);
-    }
-    return o;
-  };
-  const Offsets first = tile_offsets(0);
+  for (int s = 0; s < kPasses; ++s) {
+    const int32_t j = s * kRowsPerPass + group;
+    const uint32_t key = static_cast<uint32_t>(j < n_k - 1 ? j : n_k - 1);
+    o.k[s] = key * k_row_bytes + chunk_bytes;
+    o.v[s] = key * v_row_bytes + chunk_bytes;
+    o.bias[s] = key * static_cast<uint32_t>(p.sbn);
+  }
 
-  // Issues every load of work item (row, tile) into `slot`.
-  auto issue = [&](Slot& slot, int32_t row, int32_t tile) {
+  // Issues every load of a row into `slot`.
+  auto issue = [&](Slot& slot, int32_t row) {
     const RowCoords c = row_coords(row, p);
     const char* kp = reinterpret_cast<const char*>(p.k) + (c.b * p.sk[0] + c.h * p.sk[1]) * sizeof(T);
     const char* vp = reinterpret_cast<const char*>(p.v) + (c.b * p.sv[0] + c.h * p.sv[1]) * sizeof(T);
-    // With one tile per row (Nk <= 64) the offsets are loop invariant.
-    const Offsets o = (kSingleTile || tile == 0) ? first : tile_offsets(tile);
     // Issue order is use order: vector loads complete in order, so q, the
     // coefficient and the biases go first and K before V; the scores are
     // then computed while V is still arriving, and only the value product
     // waits for the last bytes.
-    if (tile == 0) {
-      const char* qp = reinterpret_cast<const char*>(p.q) +
-                       (c.b * p.sq[0] + c.h * p.sq[1] + c.i * p.sq[2]) * sizeof(T);
-      slot.q = load16(qp + chunk_bytes);
-      slot.scale = load_raw_scalar(p.scale, c.b * p.ssb + c.h * p.ssh, p.scale_dtype);
-    }
+    const char* qp = reinterpret_cast<const char*>(p.q) +
+                     (c.b * p.sq[0] + c.h * p.sq[1] + c.i * p.sq[2]) * sizeof(T);
+    slot.q = load16(qp + chunk_bytes);
+    slot.scale = load_raw_scalar(p.scale, c.b * p.ssb + c.h * p.ssh, p.scale_dtype);
     if (has_bias) {
       const char* bp = reinterpret_cast<const char*>(p.bias) +
                        (c.b * p.sbb + c.h * p.sbh) * bias_esize;
@@ -223,28 +212,20 @@ void rbf_stream_kernel(Problem p) {
     __builtin_amdgcn_sched_barrier(0);
   };
 
-  // Per-row running state.
-  uint4 q_raw = make_uint4(0, 0, 0, 0);
-  float q_norm = 0.f, neg_scale = 0.f, run_max = -INFINITY, run_sum = 0.f;
-  float acc[kVec];
-
-  // Reduces work item (row, tile) held in `slot`.
-  auto consume = [&](const Slot& slot, int32_t row, int32_t tile) {
-    if (tile == 0) {
-      q_raw = slot.q;
-      q_norm = reduce_low<kChunks>(dot_chunk<T>(q_raw, q_raw, 0.f), OpSum());
-      neg_scale = -decode_raw_scalar(slot.scale, p.scale_dtype);
-      run_max = -INFINITY;
-      run_sum = 0.f;
+  // Reduces the row held in `slot`.
+  auto consume = [&](const Slot& slot, int32_t row) {
+    const uint4 q_raw = slot.q;
+    const float q_norm = reduce_low<kChunks>(dot_chunk<T>(q_raw, q_raw, 0.f), OpSum());
+    const float neg_scale = -decode_raw_scalar(slot.scale, p.scale_dtype);
+    float acc[kVec];
 #pragma unroll
-      for (int e = 0; e < kVec; ++e) acc[e] = 0.f;
-    }
+    for (int e = 0; e < kVec; ++e) acc[e] = 0.f;
     float logit[kPasses];
     bool live[kPasses];
-    float tile_max = -INFINITY;
+    float row_max = -INFINITY;
 #pragma unroll
     for (int s = 0; s < kPasses; ++s) {
-      const int32_t j = tile * kWave + s * kRowsPerPass + group;
+      const int32_t j = s * kRowsPerPass + group;
       live[s] = j < n_k;
       const float dot = reduce_low<kChunks>(dot_chunk<T>(q_raw, slot.k[s], 0.f), OpSum());
       const float k_norm = reduce_low<kChunks>(dot_chunk<T>(slot.k[s], slot.k[s], 0.f), OpSum());
@@ -259,22 +240,18 @@ void rbf_stream_kernel(Problem p) {
       }
       x = live[s] ? x : -INFINITY;
       logit[s] = x;
-      tile_max = fmaxf(tile_max, x);
+      row_max = fmaxf(row_max, x);
     }
-    tile_max = reduce_high<kChunks>(tile_max, OpMax());
-    const float new_max = fmaxf(run_max, tile_max);
-    const float safe_max = new_max == -INFINITY ? 0.f : new_max;
-    const float alpha = __builtin_amdgcn_exp2f((run_max - safe_max) * kLog2e);
-    float tile_sum = 0.f;
-#pragma unroll
-    for (int e = 0; e < kVec; ++e) acc[e] *= alpha;
+    row_max = reduce_high<kChunks>(row_max, OpMax());
+    const float safe_max = row_max == -INFINITY ? 0.f : row_max;
+    float row_sum = 0.f;
     // Rows past Nk do not exist: their (clamped) values must not reach the
     // sum even as 0 * inf, so a tile with such rows zeroes them.
-    const bool ragged = (tile + 1) * kWave > n_k;
+    const bool ragged = kWave > n_k;
 #pragma unroll
     for (int s = 0; s < kPasses; ++s) {
       const float w = __builtin_amdgcn_exp2f((logit[s] - safe_max) * kLog2e);
-      tile_sum += w;
+      row_sum += w;
       uint4 vr = slot.v[s];
       if (ragged && !live[s]) vr = make_uint4(0, 0, 0, 0);
       float vf[kVec];
@@ -284,84 +261,261 @@ void rbf_stream_kernel(Problem p) {
     }
     // Each weight is replicated over the kChunks lanes of its key row; sum
     // over row groups only.
-    run_sum = run_sum * alpha + reduce_high<kChunks>(tile_sum, OpSum());
-    run_max = new_max;
-    if (tile == tiles - 1) {
-      // Sum the accumulators over row groups; lane `lane` ends with
-      // kVec / 4 finished values of its chunk, starting at element `first_e`.
-      constexpr int kOut = kVec / 4;
-      float res[kOut];
-      int first_e;
-      reduce_rows_butterfly<kChunks, kVec>(acc, res, first_e);
-      // A row whose keys are all masked has run_sum 0: 0 * inf = NaN, as eager.
-      const float inv = __builtin_amdgcn_rcpf(run_sum);
+    row_sum = reduce_high<kChunks>(row_sum, OpSum());
+    // Sum the accumulators over row groups; lane `lane` ends with
+    // kVec / 4 finished values of its chunk, starting at element `first_e`.
+    constexpr int kOut = kVec / 4;
+    float res[kOut];
+    int first_e;
+    reduce_rows_butterfly<kChunks, kVec>(acc, res, first_e);
+    // A row whose keys are all masked has row_sum 0: 0 * inf = NaN, as eager.
+    const float inv = __builtin_amdgcn_rcpf(row_sum);
 #pragma unroll
-      for (int e = 0; e < kOut; ++e) res[e] *= inv;
-      // Row groups below lane bit 16 hold copies; one of them stores.
-      if ((lane & (16 - kChunks)) == 0) {
-        const RowCoords c = row_coords(row, p);
-        store_small<OutT, kOut>(static_cast<OutT*>(p.out) + c.b * p.so[0] + c.h * p.so[1] +
-                                    c.i * p.so[2] + chunk * kVec + first_e,
-                                res);
+    for (int e = 0; e < kOut; ++e) res[e] *= inv;
+    // Row groups below lane bit 16 hold copies; one of them stores.
+    if ((lane & (16 - kChunks)) == 0) {
+      const RowCoords c = row_coords(row, p);
+      store_small<OutT, kOut>(static_cast<OutT*>(p.out) + c.b * p.so[0] + c.h * p.so[1] +
+                                  c.i * p.so[2] + chunk * kVec + first_e,
+                              res);
+    }
+  };
+
+  Slot slots[2];
+  auto row_at = [&](int r) {
+    const int32_t row = wave_id * kRows + r;
+    return row < total_rows ? row : total_rows - 1;
+  };
+  issue(slots[0], row_at(0));
+#pragma unroll
+  for (int r = 0; r < kRows; ++r) {
+    if (r + 1 < kRows) issue(slots[(r + 1) & 1], row_at(r + 1));
+    consume(slots[r & 1], row_at(r));
+  }
+}
+
+// ------------------------------------------------------------------------
+// Split kernel: few query rows over key axes of more than one 64-key tile.
+//
+// W waves (a power of two up to 16) own one query row and take its key tiles
+// in turn, so a call with few rows still has W waves per row streaming.  A
+// tile is kSplitPasses passes of the stream layout: lane l holds chunk
+// l % kChunks of key row l / kChunks of each pass (one coalesced 1 KiB wave
+// load), V in the same layout.  Each lane group of kChunks lanes keeps a
+// softmax of its own over the keys it sees (maximum, sum, value
+// accumulators), so the loop reduces nothing across groups: one merge over
+// the wave's groups and one over the row's waves (through LDS) end the row.
+//
+// Bound: HBM (K and V once each).  Two passes per tile and one tile in
+// flight per wave keep 58 registers, eight waves per SIMD, whose loads cover
+// each other's latency; a second tile in flight (87 registers, five waves)
+// and four passes (85) were no faster, and eight passes spilled.  Measured,
+// bf16, 64 subjects x 8 heads x 1000 keys of 64 dims: 22.4 us, 5.9 TB/s (a
+// plain read of the bytes: 20.3; 634 us before, on the generic kernel); 1024
+// x 8 x 128 keys of 32 dims: 22.2 us (23.2 before, as a loop of the one-tile
+// kernel), x 65 keys 13.5 (20.2).
+// ------------------------------------------------------------------------
+
+constexpr int kSplitPasses = 2;
+constexpr int kSplitMaxWaves = 16;
+
+template <typename T, typename OutT, int kChunks>
+__global__ __launch_bounds__(kSplitMaxWaves * kWave) void rbf_split_kernel(Problem p) {
+  constexpr int kVec = Vec<T>::kN;
+  constexpr int kDim = kChunks * kVec;
+  constexpr int kGroups = kWave / kChunks;      // key rows per pass
+  constexpr int kKeys = kSplitPasses * kGroups;  // key rows per tile
+  __shared__ float part_acc[kSplitMaxWaves][kDim];
+  __shared__ float part_max[kSplitMaxWaves], part_sum[kSplitMaxWaves];
+
+  args_in_sgprs(p.q, p.k, p.v, p.out, p.scale, p.bias, p.scale_dtype, p.bias_dtype, p.H, p.Nq, p.Nk);
+  args_in_sgprs(p.sq[0], p.sq[1], p.sq[2], p.sk[0], p.sk[1], p.sk[2], p.sv[0], p.sv[1], p.sv[2]);
+  args_in_sgprs(p.so[0], p.so[1], p.so[2], p.ssb, p.ssh, p.sbb, p.sbh, p.sbn, p.total_rows);
+  args_in_sgprs(p.grid_waves, p.first_row, p.nq_mul, p.nq_shift, p.h_mul, p.h_shift);
+  const int lane = threadIdx.x & (kWave - 1);
+  const int slot_wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int log_waves = p.grid_waves;
+  const int n_waves = 1 << log_waves;          // per row
+  const int wave = slot_wave & (n_waves - 1);  // of the row
+  // Workgroups are dispatched round-robin over the 8 XCDs: contiguous rows
+  // (the queries of a plane) run on one XCD and share its L2.
+  const int32_t total_rows = static_cast<int32_t>(p.total_rows);
+  const int32_t per_xcd = static_cast<int32_t>(gridDim.x >> 3);
+  const int32_t item = static_cast<int32_t>(blockIdx.x & 7) * per_xcd + static_cast<int32_t>(blockIdx.x >> 3);
+  const int32_t rows_here = static_cast<int>(blockDim.x) >> (6 + log_waves);
+  const int32_t first_row = p.first_row + item * rows_here;
+  if (first_row >= total_rows) return;  // the whole workgroup, before any barrier
+  // Waves past the last row repeat it (same bytes stored).
+  const int32_t row_id = first_row + (slot_wave >> log_waves);
+  const int32_t row = row_id < total_rows ? row_id : total_rows - 1;
+  const RowCoords c = row_coords(row, p);
+
+  const int32_t n_k = static_cast<int32_t>(p.Nk);
+  const int chunk = lane % kChunks;
+  const int group = lane / kChunks;
+  const uint32_t chunk_bytes = chunk * 16u;
+  const uint32_t k_row_bytes = static_cast<uint32_t>(p.sk[2]) * sizeof(T);
+  const uint32_t v_row_bytes = static_cast<uint32_t>(p.sv[2]) * sizeof(T);
+  const bool has_bias = p.bias != nullptr;
+  const int32_t bias_esize = p.bias_dtype == VECTRA_F32 ? 4 : 2;
+  const char* kp = reinterpret_cast<const char*>(p.k) + (c.b * p.sk[0] + c.h * p.sk[1]) * sizeof(T);
+  const char* vp = reinterpret_cast<const char*>(p.v) + (c.b * p.sv[0] + c.h * p.sv[1]) * sizeof(T);
+  const char* bp = reinterpret_cast<const char*>(p.bias) + (c.b * p.sbb + c.h * p.sbh) * bias_esize;
+  const uint32_t bias_misalign = base_misalign(bp);
+  const int32_t tiles = (n_k + kKeys - 1) / kKeys;
+
+  struct Slot {
+    uint4 k[kSplitPasses], v[kSplitPasses];
+    uint32_t bias[kSplitPasses];
+  };
+  // Issues every load of a tile; rows past Nk read row Nk - 1 and are masked.
+  auto issue = [&](Slot& slot, int32_t tile) {
+    uint32_t key[kSplitPasses];
+#pragma unroll
+    for (int s = 0; s < kSplitPasses; ++s) {
+      const int32_t j = tile * kKeys + s * kGroups + group;
+      key[s] = static_cast<uint32_t>(j < n_k - 1 ? j : n_k - 1);
+    }
+    if (has_bias) {
+#pragma unroll
+      for (int s = 0; s < kSplitPasses; ++s)
+        slot.bias[s] =
+            load_raw_scalar32(bp, bias_misalign, key[s] * static_cast<uint32_t>(p.sbn), p.bias_dtype).word;
+    }
+#pragma unroll
+    for (int s = 0; s < kSplitPasses; ++s) slot.k[s] = load16_stream(kp + (key[s] * k_row_bytes + chunk_bytes));
+#pragma unroll
+    for (int s = 0; s < kSplitPasses; ++s) slot.v[s] = load16_stream(vp + (key[s] * v_row_bytes + chunk_bytes));
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  Slot a;
+  const uint4 q_raw =
+      load16(reinterpret_cast<const char*>(p.q) + (c.b * p.sq[0] + c.h * p.sq[1] + c.i * p.sq[2]) * sizeof(T) +
+             chunk_bytes);
+  const RawScalar scale_raw = load_raw_scalar(p.scale, c.b * p.ssb + c.h * p.ssh, p.scale_dtype);
+  // The row's tile order is rotated by a hash of the row: where planes are a
+  // power of two apart, waves that walk them in step from the first tile
+  // would all be on the same few HBM channels (8192 rows of 256 keys: 41.9 us
+  // rotated, 51.2 in order).
+  const int32_t rotation = static_cast<int32_t>(__umulhi(static_cast<uint32_t>(row) * 0x9e3779b1u, tiles));
+  auto rotated = [&](int32_t t) { return t + rotation < tiles ? t + rotation : t + rotation - tiles; };
+  int32_t step = wave, tile = rotated(step);
+  if (step < tiles) issue(a, tile);
+  const float q_norm = reduce_low<kChunks>(dot_chunk<T>(q_raw, q_raw, 0.f), OpSum());
+  const float neg_scale = -decode_raw_scalar(scale_raw, p.scale_dtype);
+
+  // The lane group's softmax state.  Logits are subtracted before they are
+  // scaled to log2 units: a bias of the type's lowest value would overflow
+  // the other way round.
+  float run_max = -INFINITY, run_sum = 0.f;
+  float acc[kVec];
+#pragma unroll
+  for (int e = 0; e < kVec; ++e) acc[e] = 0.f;
+
+  auto consume = [&](const Slot& slot, int32_t t) {
+    const bool ragged = (t + 1) * kKeys > n_k;
+    float logit[kSplitPasses];
+    float tile_max = -INFINITY;
+#pragma unroll
+    for (int s = 0; s < kSplitPasses; ++s) {
+      const int32_t j = t * kKeys + s * kGroups + group;
+      const float dot = dot_chunk<T>(q_raw, slot.k[s], 0.f);
+      const float k_norm = dot_chunk<T>(slot.k[s], slot.k[s], 0.f);
+      const float part = reduce_low<kChunks>(fmaf(-2.f, dot, k_norm), OpSum());
+      const float dist = clamp_distance(q_norm + part);
+      float x = neg_scale * dist;
+      if (has_bias) {
+        const uint32_t key = static_cast<uint32_t>(j < n_k - 1 ? j : n_k - 1);
+        const uint32_t bytes = key * static_cast<uint32_t>(p.sbn) * bias_esize + bias_misalign;
+        x += decode_raw_scalar(RawScalar{slot.bias[s], (bytes & 2u) * 8u}, p.bias_dtype);
       }
+      x = j < n_k ? x : -INFINITY;
+      logit[s] = x;
+      tile_max = fmaxf(tile_max, x);
     }
-  };
-
-  auto advance = [&](int32_t& row, int32_t& tile) {
-    if (kSingleTile) {
-      row += n_waves;
-      return;
-    }
-    if (++tile == tiles) {
-      tile = 0;
-      row += n_waves;
-    }
-  };
-
-  if constexpr (kRows > 0) {
-    Slot slots[2];
-    auto row_at = [&](int r) {
-      const int32_t row = wave_id * kRows + r;
-      return row < total_rows ? row : total_rows - 1;
-    };
-    issue(slots[0], row_at(0), 0);
+    const float new_max = fmaxf(run_max, tile_max);
+    const float safe_max = new_max == -INFINITY ? 0.f : new_max;
+    const float alpha = __builtin_amdgcn_exp2f((run_max - safe_max) * kLog2e);
+    run_sum *= alpha;
 #pragma unroll
-    for (int r = 0; r < kRows; ++r) {
-      if (r + 1 < kRows) issue(slots[(r + 1) & 1], row_at(r + 1), 0);
-      consume(slots[r & 1], row_at(r), 0);
+    for (int e = 0; e < kVec; ++e) acc[e] *= alpha;
+#pragma unroll
+    for (int s = 0; s < kSplitPasses; ++s) {
+      const float w = __builtin_amdgcn_exp2f((logit[s] - safe_max) * kLog2e);
+      run_sum += w;
+      uint4 vr = slot.v[s];
+      // Rows past Nk do not exist: their (clamped) values must not reach the
+      // sum even as 0 * inf.
+      if (ragged && t * kKeys + s * kGroups + group >= n_k) vr = make_uint4(0, 0, 0, 0);
+      float vf[kVec];
+      unpack<T>(vr, vf);
+#pragma unroll
+      for (int e = 0; e < kVec; ++e) acc[e] = fmaf(w, vf[e], acc[e]);
     }
-    return;
+    run_max = new_max;
+  };
+
+  while (step < tiles) {
+    consume(a, tile);
+    step += n_waves;
+    tile = rotated(step);
+    if (step < tiles) issue(a, tile);
   }
 
-  // Two slots alternate roles, so the prefetch needs no register copies.
-  // Each branch has its own copy of the reduction: after a join of a path
-  // that issued the prefetch and one that did not, the compiler could only
-  // wait for every outstanding load, the prefetch included.
-  Slot a, b;
-  int32_t row = wave_id, tile = 0;
-  issue(a, row, tile);
-  while (true) {
-    int32_t next_row = row, next_tile = tile;
-    advance(next_row, next_tile);
-    if (next_row < total_rows) {
-      issue(b, next_row, next_tile);
-      consume(a, row, tile);
-    } else {
-      consume(a, row, tile);
-      break;
+  // Merge the wave's lane groups: a group without a live key weighs 0.
+  const float wave_max = reduce_high<kChunks>(run_max, OpMax());
+  const float mine = __builtin_amdgcn_exp2f((run_max - (wave_max == -INFINITY ? 0.f : wave_max)) * kLog2e);
+  const float wave_sum = reduce_high<kChunks>(run_sum * mine, OpSum());
+#pragma unroll
+  for (int e = 0; e < kVec; ++e) acc[e] *= mine;
+  constexpr int kOut = kChunks == 32 ? kVec / 2 : kVec / 4;
+  float res[kOut];
+  int first_e;
+  if constexpr (kChunks == 32) {  // two key rows per pass: lane bit 32 only
+#pragma unroll
+    for (int i = 0; i < kOut; ++i) {
+      const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[i]), __float_as_uint(acc[i + kOut]), false,
+                                                      false);
+      res[i] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
     }
-    row = next_row;
-    tile = next_tile;
-    advance(next_row, next_tile);
-    if (next_row < total_rows) {
-      issue(a, next_row, next_tile);
-      consume(b, row, tile);
-    } else {
-      consume(b, row, tile);
-      break;
+    first_e = (lane & 32) ? kOut : 0;
+  } else {
+    reduce_rows_butterfly<kChunks, kVec>(acc, res, first_e);
+  }
+  OutT* out = static_cast<OutT*>(p.out) + c.b * p.so[0] + c.h * p.so[1] + c.i * p.so[2];
+  // Row groups below lane bit 16 hold copies; one of them writes.
+  const bool writer = kChunks >= 16 || (lane & (16 - kChunks)) == 0;
+  if (n_waves == 1) {
+    // A row whose keys are all masked has sum 0: 0 * inf = NaN, as eager.
+    const float inv = __builtin_amdgcn_rcpf(wave_sum);
+#pragma unroll
+    for (int i = 0; i < kOut; ++i) res[i] *= inv;
+    if (writer) store_small<OutT, kOut>(out + chunk * kVec + first_e, res);
+    return;
+  }
+  if (writer) {
+#pragma unroll
+    for (int i = 0; i < kOut; ++i) part_acc[slot_wave][chunk * kVec + first_e + i] = res[i];
+  }
+  if (lane == 0) {
+    part_max[slot_wave] = wave_max;
+    part_sum[slot_wave] = wave_sum;
+  }
+  __syncthreads();
+  const int w0 = slot_wave & -n_waves;  // the row's first wave
+  const int d = static_cast<int>(threadIdx.x) - w0 * kWave;
+  if (d < kDim) {
+    float m = -INFINITY;
+    for (int w = 0; w < n_waves; ++w) m = fmaxf(m, part_max[w0 + w]);
+    const float safe = m == -INFINITY ? 0.f : m;
+    float sum = 0.f, value = 0.f;
+    for (int w = 0; w < n_waves; ++w) {
+      const float f = __builtin_amdgcn_exp2f((part_max[w0 + w] - safe) * kLog2e);
+      sum = fmaf(f, part_sum[w0 + w], sum);
+      value = fmaf(f, part_acc[w0 + w][d], value);
     }
-    row = next_row;
-    tile = next_tile;
+    out[d] = from_float<OutT>(value * __builtin_amdgcn_rcpf(sum));
   }
 }
 
@@ -502,18 +656,43 @@ static hipError_t launch_stream_k(Problem& p, hipStream_t s) {
                 dim3(256), p, s);
 }
 
+// Waves per row: enough for 8 waves per CU over all rows (two per SIMD; from
+// there on more waves per row only add merges: 2048 rows of 65-400 keys ran
+// 0-50% slower with two to eight), at most one per key tile.  Measured with 1
+// / 2 / 4 / 8 / 16 waves: 8 rows of 2048 keys 98.7 / 48.6 / 23.3 / 14.7 /
+// 12.4 us, 512 rows of 1000 keys 54.5 / 31.2 / 22.3 / 22.4 / 22.6 us, 8192
+// rows of 65 keys 13.5 / 14.0 / 17.3 / 29.5 us.
+template <typename T, typename OutT, int kChunks>
+static hipError_t launch_split(Problem& p, hipStream_t s) {
+  constexpr int kKeys = kSplitPasses * (kWave / kChunks);
+  const int64_t tiles = (p.Nk + kKeys - 1) / kKeys;
+  const int64_t slots = static_cast<int64_t>(p.compute_units) * 8;
+  int log_waves = 0;
+  while ((1 << log_waves) < kSplitMaxWaves && (2 << log_waves) <= tiles && (p.total_rows << log_waves) < slots)
+    ++log_waves;
+  const int rows_here = log_waves < 2 ? 4 >> log_waves : 1;
+  p.grid_waves = log_waves;
+  // A grid holds fewer than 2^32 threads, so very many rows (of one wave
+  // each) take several launches.
+  constexpr int64_t kMaxRows = int64_t{1} << 25;
+  for (int64_t row = 0; row < p.total_rows; row += kMaxRows) {
+    const int64_t rows = p.total_rows - row < kMaxRows ? p.total_rows - row : kMaxRows;
+    const int64_t items = (rows + rows_here - 1) / rows_here;
+    p.first_row = static_cast<int32_t>(row);
+    const dim3 grid(static_cast<unsigned>((items + 7) / 8 * 8));
+    const hipError_t err = launch(reinterpret_cast<const void*>(&rbf_split_kernel<T, OutT, kChunks>), grid,
+                                  dim3(static_cast<unsigned>(rows_here << (log_waves + 6))), p, s);
+    if (err != hipSuccess) return err;
+  }
+  return hipSuccess;
+}
+
 // Rows per wave for one-tile rows: about `budget` waves, at most kMaxRows
 // rows each (the register footprint of two slots bounds it for wide heads).
 template <typename T, typename OutT, int kChunks, int kMaxRows>
 static hipError_t launch_stream_c(Problem& p, hipStream_t s) {
+  if (p.Nk > kWave) return launch_split<T, OutT, kChunks>(p, s);
   const int64_t budget = p.grid_waves;
-  // Rows of 8 or 16 chunks with several key tiles would spill registers in
-  // the looping variant: the host sends them to another kernel instead.
-  if (kChunks >= 8 && p.Nk > kWave) return hipErrorInvalidValue;
-  if (kChunks < 8 && p.Nk > kWave) {
-    p.grid_waves = static_cast<int32_t>(p.total_rows < budget ? p.total_rows : budget);
-    return launch_stream_k<T, OutT, kChunks, (kChunks < 8 ? 0 : 1)>(p, s);
-  }
   const int64_t rows = p.total_rows;
   int rows_per_wave = rows > 2 * budget ? 4 : (rows > budget ? 2 : 1);
   if (rows_per_wave > kMaxRows) rows_per_wave = kMaxRows;
@@ -532,6 +711,9 @@ static hipError_t launch_stream_t(Problem& p, int chunks, hipStream_t s) {
     case 4: return launch_stream_c<T, OutT, 4, 4>(p, s);
     case 8: return launch_stream_c<T, OutT, 8, 4>(p, s);
     case 16: return launch_stream_c<T, OutT, 16, 1>(p, s);
+    case 32:  // 128-dim fp32 heads: any key count (a 64-key tile would spill)
+      if constexpr (sizeof(T) == 4) return launch_split<T, OutT, 32>(p, s);
+      return hipErrorInvalidValue;
     default: return hipErrorInvalidValue;
   }
 }

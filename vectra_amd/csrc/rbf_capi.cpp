@@ -155,10 +155,9 @@ int stream_chunks(const vectra_rbf_args* a) {
   const int vec = 16 / in_sz;
   if (a->head_dim != a->value_dim || a->head_dim == 0 || a->head_dim % vec != 0) return 0;
   const int64_t chunks = a->head_dim / vec;
-  if (chunks != 2 && chunks != 4 && chunks != 8 && chunks != 16) return 0;
-  // 8- and 16-chunk rows run one key tile per row only (more would spill
-  // registers in the looping variant).
-  if (chunks >= 8 && a->n_k > 64) return 0;
+  // 32 chunks: 128-dim fp32 heads.
+  const bool wide = chunks == 32 && in_sz == 4 && a->n_k > 0;
+  if (chunks != 2 && chunks != 4 && chunks != 8 && chunks != 16 && !wide) return 0;
   // Per-lane key offsets inside a (b, h) plane are unsigned 32-bit: key row
   // strides (K, V and the bias) must be non-negative and the last row's
   // bytes within 2^31.

@@ -31,6 +31,7 @@ struct Problem {
   int32_t grid_waves;  // waves launched by persistent kernels (<= total_rows)
   int32_t compute_units;  // of the device the launch runs on
   int32_t flags;          // VECTRA_FLAG_* bits
+  int32_t first_row;      // split kernel: first query row of this launch
   uint32_t nq_mul, nq_shift;  // FastDiv of Nq (see fast_div)
   uint32_t h_mul, h_shift;    // FastDiv of H
 };

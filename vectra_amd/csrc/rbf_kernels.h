@@ -11,9 +11,10 @@ struct Problem;
 // Multiplier and shift for fast_div (division of 31-bit values by d >= 1).
 void make_fast_div(int64_t d, uint32_t* mul, uint32_t* shift);
 
-// Stream kernel: requires unit element stride in d for q, k, v and out,
-// 16-byte-aligned rows, D == Dv == chunks * (16 / sizeof(input element)),
-// chunks in {2, 4, 8, 16}.
+// Stream kernels (one key tile, or the waves of a row sharing its tiles):
+// require unit element stride in d for q, k, v and out, 16-byte-aligned rows,
+// D == Dv == chunks * (16 / sizeof(input element)), chunks in {2, 4, 8, 16},
+// or 32 with fp32 and Nk >= 1.
 hipError_t launch_stream(Problem& p, int in_dtype, int out_dtype, int chunks, hipStream_t s);
 
 // Generic kernel: any strides and sizes.  Its grid has one row of
