@@ -180,16 +180,21 @@ typedef struct vectra_scan_top_k_args {
 int vectra_scan_top_k(const vectra_scan_top_k_args* args, hipStream_t stream);
 
 /*
- * vectra_scan_top_k with a device workspace: below 64 queries the
- * candidates of a query are cut into ranges, one workgroup each (at least 64
- * candidates per range, at most 64 ranges, ranges * k <= 2048), and the
- * workgroup that finishes last merges the ranges' k best; the results are
- * the same bits as vectra_scan_top_k's.  The workspace is `workspace_bytes`
- * of device memory, 256-byte aligned, whose first 256 bytes (arrival
- * counters) are zero before the first call on it; every call leaves them
- * zero.  With a NULL or smaller workspace than
- * vectra_scan_top_k_workspace_bytes(args), or 64 queries or more, this is
- * vectra_scan_top_k.  Calls that share a workspace must not overlap.
+ * vectra_scan_top_k with a device workspace; the results are the same bits
+ * as vectra_scan_top_k's.  Four queries or more over 4,096 candidates or more
+ * (and 12 queries or 131,072 pairs, dimension a multiple of 4 up to 256,
+ * 16-byte-aligned rows, k at most 512) are filtered: the matrix cores bound
+ * every distance, and only candidates that can be among the k nearest are
+ * computed.  Other calls of fewer than 64 queries have the candidates of a
+ * query cut into ranges, one workgroup each (at least 64 candidates per
+ * range, at most 64 ranges, ranges * k <= 2048), and the workgroup that
+ * finishes last merges the ranges' k best.  The workspace is
+ * `workspace_bytes` of device memory, 256-byte aligned, whose first 256 bytes
+ * (arrival counters) are zero before the first call on it; every call leaves
+ * them zero.  With a smaller workspace than
+ * vectra_scan_top_k_workspace_bytes(args) the ranges are used if their keys
+ * fit it; without that, this is vectra_scan_top_k.  Calls that share a
+ * workspace must not overlap.
  * Replaces the same reference loop as vectra_scan_top_k
  * (shard_index.cc:236-264), for requests of one or a few queries.
  */

@@ -698,6 +698,31 @@ __device__ __forceinline__ uint64_t wave_min(uint64_t key) {
   return key;
 }
 
+// Sorts keys[0 .. k + n) in LDS ascending (padded with empty slots to a power
+// of two), leaving the k best in keys[0 .. k); every thread of the workgroup
+// takes part.
+template <int kSortThreads>
+__device__ __forceinline__ void sort_keys(uint64_t* keys, int k, int n, int tid) {
+  int size = 2;
+  while (size < k + n) size <<= 1;
+  for (int i = k + n + tid; i < size; i += kSortThreads) keys[i] = kNoKey;
+  __syncthreads();
+  for (int span = 2; span <= size; span <<= 1) {
+    for (int stride = span >> 1; stride > 0; stride >>= 1) {
+      for (int t = tid; t < size / 2; t += kSortThreads) {
+        const int i = 2 * t - (t & (stride - 1));
+        const int j = i + stride;
+        const uint64_t a = keys[i], b = keys[j];
+        if ((a > b) == ((i & span) == 0)) {
+          keys[i] = b;
+          keys[j] = a;
+        }
+      }
+      __syncthreads();
+    }
+  }
+}
+
 // kTopKThreads threads; a 16-lane group loads kTopKCands candidates at once,
 // kSteps times per round of candidates between merge checks.  kDim is the
 // row dimension when known at compile time (a multiple of 16 up to 128: the
@@ -727,28 +752,7 @@ __global__ __launch_bounds__(kTopKThreads) void scan_top_k_kernel(TopK p) {
   if (tid == 0) fill = 0;
   __syncthreads();
 
-  // Sorts keys[0 .. k + n) ascending (padded with empty slots to a power of
-  // two), leaving the k best in keys[0 .. k); every thread takes part.
-  auto merge = [&](int n) {
-    int size = 2;
-    while (size < k + n) size <<= 1;
-    for (int i = k + n + tid; i < size; i += kTopKThreads) keys[i] = kNoKey;
-    __syncthreads();
-    for (int span = 2; span <= size; span <<= 1) {
-      for (int stride = span >> 1; stride > 0; stride >>= 1) {
-        for (int t = tid; t < size / 2; t += kTopKThreads) {
-          const int i = 2 * t - (t & (stride - 1));
-          const int j = i + stride;
-          const uint64_t a = keys[i], b = keys[j];
-          if ((a > b) == ((i & span) == 0)) {
-            keys[i] = b;
-            keys[j] = a;
-          }
-        }
-        __syncthreads();
-      }
-    }
-  };
+  auto merge = [&](int n) { sort_keys<kTopKThreads>(keys, k, n, tid); };
 
   // The first selection of a workgroup whose rounds hold at most a wave's
   // worth of candidates: nothing has been selected yet, so keys[0 .. k) are
@@ -1018,6 +1022,8 @@ __global__ __launch_bounds__(kTopKThreads) void scan_top_k_kernel(TopK p) {
   }
 }
 
+#include "top_k_filter.h"
+
 }  // namespace
 }  // namespace vectra_scan
 
@@ -1255,6 +1261,131 @@ int launch_top_k(int64_t queries, TopK& p, hipStream_t stream) {
                                   stream));
 }
 
+// The filtered form (top_k_filter.h) for valid parameters: its launch shapes
+// and workspace, or bytes 0 where it does not apply.
+struct FilterPlan {
+  TopKFilter f;
+  int64_t query_blocks = 0, bytes = 0;
+  int64_t minima = 0, limit = 0, counts = 0, lists = 0;  // byte offsets
+};
+
+// The filtered form's four launches take 20-23 us however small the call; the
+// exact forms about 10 us and 1.2 us more per query (one workgroup each), and
+// more with the candidates.  Measured, 128 dimensions, k = 10, exact and
+// filtered us: 12 queries x 4,096 27 and 23, 8 x 4,096 20 and 23, 8 x 16,384
+// 25 and 22, 4 x 32,768 24 and 25, 4 x 65,536 34 and 27, 64 x 4,096 78 and 25.
+// Below four queries the split form keeps its small workspace.
+constexpr int64_t kFilterMinQueries = 4;
+constexpr int64_t kFilterMinCands = 4096;
+constexpr int64_t kFilterQueriesAlone = 12;       // from here on whatever the candidates
+constexpr int64_t kFilterMinPairs = int64_t{1} << 17;  // below: this many (query, candidate) pairs
+
+FilterPlan top_k_filter_plan(int64_t queries, const TopK& p) {
+  FilterPlan plan;
+  if (queries < kFilterMinQueries || p.num_cand < kFilterMinCands || p.num_cand > 0x7fffffffLL ||
+      (queries < kFilterQueriesAlone && queries * p.num_cand < kFilterMinPairs) || p.num_rows < 1 ||
+      p.k > kFilterMaxK || p.dim < 4 || p.dim > kFilterMaxDim || p.dim % 4 != 0 || p.row_stride % 4 != 0 ||
+      reinterpret_cast<uintptr_t>(p.rows) % 16 != 0)
+    return plan;
+  const int64_t blocks = (queries + kFilterQueries - 1) / kFilterQueries;
+  if (blocks > kMaxBlocksY) return plan;
+  TopKFilter& f = plan.f;
+  f.t = p;
+  f.num_queries = queries;
+  f.tiles = static_cast<int32_t>((p.num_cand + kFilterTile - 1) / kFilterTile);
+  // The sample: about 4,096 waves over all query blocks, a group of
+  // candidates each, or four where that gives less than 8 groups per result
+  // (the k-th smallest minimum is then near the k-th smallest bound).
+  int64_t waves = 4096 / blocks;
+  waves = waves > 1024 ? 1024 : (waves < 64 ? 64 : waves);
+  if (waves > f.tiles) waves = f.tiles;
+  f.group_cols = waves >= 8 * p.k ? 1 : 4;
+  if (f.group_cols == 4) {
+    waves = 2 * p.k > 256 ? 2 * p.k : 256;
+    if (waves > f.tiles) waves = f.tiles;
+  }
+  if (waves * f.group_cols < 3 * p.k || waves * f.group_cols > kFilterMaxGroups) return plan;
+  f.sample_waves = static_cast<int32_t>(waves);
+  // A quarter of the candidates; half where many results are wanted, whose
+  // surviving pairs then cost more than the sample does (1,024 queries, 12,500
+  // rows, k = 100: 121 us with a quarter, 87 with half; 8 queries, 500,000
+  // rows: 49 and 53).
+  const int64_t share = queries * p.k >= 16384 ? 2 : 4;
+  const int64_t each = (f.tiles / share + waves - 1) / waves;
+  f.sample_tiles = static_cast<int32_t>(each < 1 ? 1 : (each * waves > f.tiles ? f.tiles / waves : each));
+  f.sample_step = static_cast<int32_t>(f.tiles / (waves * f.sample_tiles));
+  // The filter: up to 768 workgroups (three per CU, all resident at once), at
+  // least one per two results, so that a workgroup's share of the k nearest
+  // is a few.
+  int64_t wgs = 768 / blocks;
+  if (wgs < p.k / 2) wgs = p.k / 2;
+  if (wgs < 1) wgs = 1;
+  const int64_t per_wave = (f.tiles + wgs * kFilterWaves - 1) / (wgs * kFilterWaves);
+  if (per_wave >= 1 << 22) return plan;
+  f.workgroups = static_cast<int32_t>((f.tiles + per_wave * kFilterWaves - 1) / (per_wave * kFilterWaves));
+  const int64_t padded = blocks * kFilterQueries;
+  auto take = [&](int64_t bytes) {
+    const int64_t at = plan.bytes;
+    plan.bytes += (bytes + 255) / 256 * 256;
+    return at;
+  };
+  plan.query_blocks = blocks;
+  take(kCounterBytes);  // the split form's counters stay as they are
+  plan.minima = take(padded * waves * f.group_cols * static_cast<int64_t>(sizeof(float)));
+  plan.limit = take(padded * static_cast<int64_t>(sizeof(float)));
+  plan.counts = take(padded * f.workgroups * static_cast<int64_t>(sizeof(uint32_t)));
+  plan.lists = take(padded * f.workgroups * kFilterCap * static_cast<int64_t>(sizeof(uint64_t)));
+  return plan;
+}
+
+template <bool kIds, int kChunks, int kTiles>
+int launch_top_k_filter(FilterPlan& plan, hipStream_t stream) {
+  TopKFilter& f = plan.f;
+  void* args[] = {&f};
+  const unsigned blocks = static_cast<unsigned>(plan.query_blocks);
+  const int slabs = (f.t.dim + 32 * kChunks - 1) / (32 * kChunks);
+  const size_t lds = static_cast<size_t>(slabs) * kChunks * kTiles * kWaveLanes * 16;
+  auto go = [&](const void* kernel, dim3 grid, size_t bytes, unsigned threads = kFilterThreads) {
+    return launched(hipLaunchKernel(kernel, grid, dim3(threads), args, bytes, stream));
+  };
+  int st = go(reinterpret_cast<const void*>(&top_k_bound_kernel<kIds, kChunks, kTiles, true>),
+              dim3((f.sample_waves + kFilterWaves - 1) / kFilterWaves, blocks), lds);
+  if (st == VECTRA_SCAN_OK)
+    st = go(f.sample_waves * f.group_cols <= 1024
+                ? reinterpret_cast<const void*>(&top_k_limit_kernel<1024 / kWaveLanes>)
+                : reinterpret_cast<const void*>(&top_k_limit_kernel<kFilterMaxGroups / kWaveLanes>),
+            dim3(kFilterQueries / kFilterWaves, blocks), 0);
+  if (st == VECTRA_SCAN_OK)
+    st = go(reinterpret_cast<const void*>(&top_k_bound_kernel<kIds, kChunks, kTiles, false>), dim3(f.workgroups, blocks), lds);
+  if (st == VECTRA_SCAN_OK)
+    // A thread per list where that takes one pass over the lists.
+    st = f.workgroups > 256
+             ? go(reinterpret_cast<const void*>(&top_k_merge_kernel<kIds, 1024>),
+                  dim3(static_cast<unsigned>(f.num_queries)), 0, 1024)
+             : go(reinterpret_cast<const void*>(&top_k_merge_kernel<kIds, 256>),
+                  dim3(static_cast<unsigned>(f.num_queries)), 0, 256);
+  return st;
+}
+
+template <int kChunks, int kTiles>
+int launch_top_k_filter(FilterPlan& plan, hipStream_t stream) {
+  return plan.f.t.ids != nullptr ? launch_top_k_filter<true, kChunks, kTiles>(plan, stream)
+                                 : launch_top_k_filter<false, kChunks, kTiles>(plan, stream);
+}
+
+// Runs the filtered form on a workspace of at least plan.bytes.
+int run_top_k_filter(FilterPlan& plan, void* workspace, hipStream_t stream) {
+  char* base = static_cast<char*>(workspace);
+  TopKFilter& f = plan.f;
+  f.minima = reinterpret_cast<float*>(base + plan.minima);
+  f.limit = reinterpret_cast<float*>(base + plan.limit);
+  f.counts = reinterpret_cast<uint32_t*>(base + plan.counts);
+  f.lists = reinterpret_cast<uint64_t*>(base + plan.lists);
+  const bool few = f.num_queries <= 16;
+  if (f.t.dim <= 64) return few ? launch_top_k_filter<2, 1>(plan, stream) : launch_top_k_filter<2, 4>(plan, stream);
+  return few ? launch_top_k_filter<4, 1>(plan, stream) : launch_top_k_filter<4, 4>(plan, stream);
+}
+
 // Points the split form at a workspace: counters first, keys after.
 void use_workspace(TopK& p, int64_t splits, void* base) {
   p.splits = static_cast<int32_t>(splits);
@@ -1293,6 +1424,8 @@ extern "C" int vectra_scan_top_k(const vectra_scan_top_k_args* a, hipStream_t st
 extern "C" int64_t vectra_scan_top_k_workspace_bytes(const vectra_scan_top_k_args* a) {
   TopK p;
   if (top_k_params(a, p) != VECTRA_SCAN_OK) return 0;
+  const FilterPlan plan = top_k_filter_plan(a->num_queries, p);
+  if (plan.bytes > 0) return plan.bytes;
   return top_k_workspace(a->num_queries, top_k_splits(a->num_queries, p), p.k);
 }
 
@@ -1303,6 +1436,9 @@ extern "C" int vectra_scan_top_k_ws(const vectra_scan_top_k_args* a, void* works
   if (st != VECTRA_SCAN_OK || a->num_queries == 0) return st;
   if (workspace != nullptr && (reinterpret_cast<uintptr_t>(workspace) & 255u) != 0)
     return VECTRA_SCAN_INVALID_ARGUMENT;
+  FilterPlan plan = top_k_filter_plan(a->num_queries, p);
+  if (plan.bytes > 0 && workspace != nullptr && workspace_bytes >= plan.bytes)
+    return run_top_k_filter(plan, workspace, stream);
   const int64_t splits = top_k_splits(a->num_queries, p);
   if (splits > 1 && workspace != nullptr && workspace_bytes >= top_k_workspace(a->num_queries, splits, p.k))
     use_workspace(p, splits, workspace);

@@ -284,10 +284,11 @@ def nearest(queries: torch.Tensor, rows: torch.Tensor, k: int, ids=None, out=Non
     tensors (contiguous, of those shapes and dtypes).
 
     `form` picks the entry point, all with the same results: 'split'
-    (vectra_scan_top_k_ws: below 64 queries a query's candidates are spread
-    over several workgroups; `workspace` is a uint8 CUDA tensor of at least
+    (vectra_scan_top_k_ws: several queries over many candidates are filtered
+    by distance bounds, a few queries' candidates spread over several
+    workgroups; `workspace` is a uint8 CUDA tensor of at least
     workspace_bytes(...) whose first 256 bytes are zero before its first use,
-    or None to allocate a zeroed one), 'single' (vectra_scan_top_k, one
+    or None to allocate one), 'single' (vectra_scan_top_k, one
     workgroup per query) or 'no_alloc' (vectra_scan_top_k_no_alloc, the
     split form on the library's own scratch)."""
     if form not in TOP_K_FORMS:
@@ -304,7 +305,8 @@ def nearest(queries: torch.Tensor, rows: torch.Tensor, k: int, ids=None, out=Non
         else:
             need = int(lib.vectra_scan_top_k_workspace_bytes(ctypes.byref(args)))
             if workspace is None:
-                workspace = torch.zeros(max(need, 1), dtype=torch.uint8, device=device)
+                workspace = torch.empty(max(need, 256), dtype=torch.uint8, device=device)
+                workspace[:256].zero_()  # the arrival counters
             _on_gpu(workspace, 'workspace')
             if workspace.dtype != torch.uint8 or not workspace.is_contiguous():
                 raise ValueError('workspace must be a contiguous uint8 tensor')
