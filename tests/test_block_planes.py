@@ -1,0 +1,101 @@
+"""16-bit planes beyond one tile with a key bias or query counts that split
+unevenly: planes staged whole in LDS (up to 160 KB: 310 to 1,024 keys by head
+width) and streamed key tiles, at the sizes where the staging, the key pairs,
+the waves and the work items end (GPU, through the C ABI)."""
+
+import math
+
+import pytest
+import torch
+
+from oracle import rbf as oracle
+from vectra_amd.kernels import capi
+
+pytestmark = pytest.mark.gpu
+
+GATE = {'rtol': 1e-3, 'atol': 1e-4}
+LOWEST = torch.finfo(torch.float32).min
+
+
+def _inputs(batch, heads, n_q, n_k, dim, dtype, seed):
+    g = torch.Generator().manual_seed(seed)
+    q, k, v = (torch.randn(batch, n, heads, dim, generator=g).to(dtype).transpose(1, 2) for n in (n_q, n_k, n_k))
+    scale = (0.5 + torch.rand(1, heads, 1, 1, generator=g)) / dim
+    counts = torch.randint(1, n_k + 1, (batch, 1, 1, 1), generator=g)
+    bias = torch.zeros(batch, 1, 1, n_k).masked_fill(torch.arange(n_k) >= counts, -math.inf)
+    return q, k, v, scale, bias
+
+
+def _run(q, k, v, scale, bias, variant='tile'):
+    # Head-transposed views keep their strides on the device.
+    dev = [t.transpose(1, 2).contiguous().cuda().transpose(1, 2) for t in (q, k, v)]
+    got = capi.forward(*dev, scale.cuda(), None if bias is None else bias.cuda(), out_dtype=torch.float32,
+                       variant=variant)
+    torch.cuda.synchronize()
+    return got.cpu().double()
+
+
+# 64 dims: 630 keys fit (4 waves up to 157, 8 up to 314, 16 above); 32 dims:
+# all up to 1,024; 128 dims: 317.  Longer planes stream.
+@pytest.mark.parametrize('n_q,n_k,dim', [(16, 1, 64), (17, 31, 64), (33, 32, 64), (81, 33, 64), (100, 150, 64),
+                                         (257, 257, 64), (65, 315, 64), (20, 608, 64), (130, 641, 64), (300, 1023, 64),
+                                         (18, 81, 32), (129, 300, 32), (260, 1000, 32), (40, 1024, 32), (70, 1030, 32),
+                                         (16, 40, 128), (90, 130, 128), (33, 288, 128), (140, 330, 128)])
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16], ids=str)
+def test_masked_planes_against_the_float64_chain(n_q, n_k, dim, dtype):
+    q, k, v, scale, bias = _inputs(2, 3, n_q, n_k, dim, dtype, n_q + n_k)
+    print(f'masked planes: {n_q}x{n_k}x{dim} {dtype}', flush=True)
+    want = torch.from_numpy(oracle.direct_fp64(q, k, v, scale, bias))
+    torch.testing.assert_close(_run(q, k, v, scale, bias), want, **GATE)
+    # Dead key pairs are skipped: a finite bias no weight survives keeps them.
+    kept = torch.where(bias == -math.inf, torch.tensor(-1e30), bias)
+    torch.testing.assert_close(_run(q, k, v, scale, kept), want, **GATE)
+
+
+@pytest.mark.parametrize('n_k,dim', [(200, 64), (700, 64), (150, 32), (200, 128), (400, 128)])
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16], ids=str)
+@pytest.mark.parametrize('case', ['additive', 'large', 'rising', 'first_masked', 'negative_scale', 'far', 'lowest'])
+def test_biases_that_move_the_shift(case, n_k, dim, dtype):
+    """Weights shifted by the first keys' largest logits: biases around 0, far
+    from 0, rising along the keys (the range check then fails and the exact
+    passes run), with the first keys masked, gamma < 0, far points, and a mask
+    of the type's lowest value."""
+    q, k, v, scale, _ = _inputs(2, 2, 40, n_k, dim, dtype, n_k)
+    g = torch.Generator().manual_seed(5)
+    bias = torch.zeros(2, 2, 1, n_k)
+    if case == 'additive':
+        bias = torch.randn(2, 2, 1, n_k, generator=g)
+    elif case == 'large':
+        bias = 40 * torch.randn(2, 2, 1, n_k, generator=g)
+    elif case == 'rising':
+        bias = torch.linspace(-60, 60, n_k).expand(2, 2, 1, n_k)
+    elif case == 'first_masked':
+        bias[..., : n_k // 2] = -math.inf
+    elif case == 'negative_scale':
+        scale = -scale / 8
+    elif case == 'far':
+        q, k, scale = (3 * q.float()).to(dtype), (3 * k.float()).to(dtype), torch.full_like(scale, 0.3)
+    elif case == 'lowest':
+        bias[..., n_k // 3:] = LOWEST
+    print(f'shift: {case} {n_k}x{dim} {dtype}', flush=True)
+    want = torch.from_numpy(oracle.direct_fp64(q, k, v, scale, bias))
+    got = _run(q, k, v, scale, bias.contiguous())
+    generic = _run(q, k, v, scale, bias.contiguous(), 'generic')
+    # Logits of hundreds carry 2^-24 of themselves into the weights: as far
+    # from float64 as four times the general path is, where that is more.
+    allow = GATE['atol'] + GATE['rtol'] * want.abs() + 4 * (generic - want).abs().amax()
+    assert bool(((got - want).abs() <= allow).all())
+
+
+@pytest.mark.parametrize('n_k,dim', [(200, 64), (700, 64), (100, 32)])
+def test_planes_without_a_live_key_and_non_finite_masked_rows(n_k, dim):
+    q, k, v, scale, bias = _inputs(3, 2, 50, n_k, dim, torch.bfloat16, 3)
+    bias[:] = 0
+    bias[1] = -math.inf            # no live key: NaN
+    bias[2, ..., 40:] = -math.inf
+    v[2, 0, n_k - 1, 5] = math.inf  # 0 times inf: that value dim is NaN
+    k[2, 1, n_k - 2, 0] = math.nan  # a NaN distance: every row is NaN
+    got = _run(q, k, v, scale, bias)
+    assert bool(got[1].isnan().all()) and not bool(got[0].isnan().any())
+    assert bool(got[2, 0, :, 5].isnan().all()) and int(got[2, 0].isnan().sum()) == 50
+    assert bool(got[2, 1].isnan().all())

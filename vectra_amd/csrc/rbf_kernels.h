@@ -34,8 +34,8 @@ hipError_t launch_mfma(Problem& p, int in_dtype, int out_dtype, hipStream_t s);
 bool plane_supports(const Problem& p, int in_dtype, int out_dtype);
 hipError_t launch_plane(Problem& p, int in_dtype, int out_dtype, hipStream_t s);
 
-// Tile kernel (key tiles streamed through LDS, 32 query rows per wave):
-// bf16/fp16 inputs, output in the input dtype or fp32, D == Dv in
+// Tile kernels (planes whose keys fit LDS staged whole, key tiles streamed
+// through LDS beyond): bf16/fp16 inputs, output in the input dtype or fp32, D == Dv in
 // {32, 64, 128}, unit d stride, 16-byte-aligned rows.
 bool tile_supports(const Problem& p, int in_dtype, int out_dtype);
 hipError_t launch_tile(Problem& p, int in_dtype, int out_dtype, hipStream_t s);

@@ -24,10 +24,17 @@
 //    operand sums the same hi + lo weights the values are weighted by.
 // Without a bias and with gamma >= 0, x <= 0 (d >= 0 up to rounding), so
 // exp2(x) is used as the weight directly: one pass over the keys, no running
-// maximum and no rescaling.  If a query's weight sum then ends below the
-// range in which the 16-bit split is accurate (the query is far from every
-// key), and always with a bias or gamma < 0, the item is computed exactly:
-// one pass finds each query's largest logit, a second subtracts it.
+// maximum and no rescaling.  With a bias, one pass too: each query's weights
+// are shifted by its largest logit over the first tile.  If a query's weight
+// sum then ends outside the range in which the 16-bit split is accurate (the
+// query is far from every key, later keys weigh far more than the first), and
+// always for gamma < 0 without a bias, the item is computed exactly: one pass
+// finds each query's largest logit, a second subtracts it.  (The kernel is
+// built with and without a bias: neither carries the other's passes.)
+// With a bias, key pairs whose keys are all masked are skipped, as in
+// rbf_block_impl.h, which takes the planes whose keys fit LDS.  Measured, 128
+// planes of 1000 x 1000 x 64 bf16 with half the keys masked: 94.5 us with two
+// passes over every key, 67.2 now.
 // Weights are fed to the second product as hi + lo 16-bit pairs (~2^-17 of
 // each weight).  The distance is not clamped at zero: where rounding makes
 // the expansion negative, -d and the reference's max(d, 0) = 0 are both
@@ -74,7 +81,9 @@
 
 #include "rbf_common.h"
 #include "rbf_kernels.h"
+#include "rbf_block_impl.h"
 #include "rbf_mfma_ops.h"
+#include "rbf_tile_ops.h"
 
 namespace vectra {
 
@@ -137,7 +146,7 @@ constexpr float kFastWalk = kFastSigmas * 0x1p-11f * 0.57735026919f;  // kFastSi
 // K and V^T fragment, and each tile's staging, then serve 64 queries per
 // wave: 10 % faster at config 4 than two blocks at three waves); 128-dim
 // heads keep two blocks at two waves.
-template <typename T, typename OutT, int kD, int kKeys, int kWaves, int kCB>
+template <typename T, typename OutT, int kD, int kKeys, int kWaves, int kCB, bool kBias>
 __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kD <= 64 && kCB <= 2 ? 3 : 2))) void
 rbf_tile_kernel(Problem p, int32_t q_blocks) {
   using G = TileGeo<T, kD, kKeys, kWaves, kCB>;
@@ -155,17 +164,26 @@ rbf_tile_kernel(Problem p, int32_t q_blocks) {
   // below 2^-21 of a sum of at least 2^-3.
   constexpr bool kBf16 = __is_same(T, __bf16);
   constexpr float kSumLo = kBf16 ? 0x1p-32f : 0x1p-3f;
+  // Weights above 1 (a pass shifted by a part of the keys): each stays inside
+  // fp16 up to this sum, and bf16 values overflow the products only above
+  // 2^96, which the pass checks for.
+  constexpr float kSumHi = kBf16 ? 0x1p32f : 0x1p15f;
   typedef _Float16 h2v __attribute__((ext_vector_type(2)));
   // Fast pass statistic: the largest |v| this thread staged in the pass (fp32
   // for bf16 inputs, packed fp16 for fp16 inputs).
   float vmax = 0.f;
   h2v vmax16 = {0, 0};
+  bool any_live = false;  // with a bias: this thread staged a key that is not masked
 
   extern __shared__ __align__(16) unsigned char lds[];
   __shared__ int32_t exact_flag[2];
-  __shared__ int32_t split_flag[2];  // the fast pass did not hold
+  __shared__ int32_t split_flag[2];  // no bias: the fast pass did not hold
   __shared__ float vmax_wave[2][kWaves];  // the fast pass's max |v| per wave
   __shared__ int32_t abort_flag[2];  // the fast pass was abandoned early
+  __shared__ int32_t live_flag[2];   // some key of the plane is not masked
+  // With a bias: whether each staged piece (a wave's 64 / kChunks keys of one
+  // slot) of a buffer holds a key that can weigh or a non-finite value.
+  __shared__ __align__(8) uint8_t piece_live[2][G::kSlots * kWaves];
 
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
@@ -177,7 +195,6 @@ rbf_tile_kernel(Problem p, int32_t q_blocks) {
   const int32_t n_k = static_cast<int32_t>(p.Nk);
   const int32_t items = static_cast<int32_t>(p.B * p.H) * q_blocks;
   const int32_t tiles = (n_k + kKeys - 1) / kKeys;
-  const bool has_bias = p.bias != nullptr;
   const int32_t bias_esize = p.bias_dtype == VECTRA_F32 ? 4 : 2;
   const uint32_t q_row_bytes = static_cast<uint32_t>(p.sq[2]) * 2u;
   const uint32_t k_row_bytes = static_cast<uint32_t>(p.sk[2]) * 2u;
@@ -214,7 +231,7 @@ rbf_tile_kernel(Problem p, int32_t q_blocks) {
   // loads over the plane's rows, so rows past Nk read zeros (or, where rows
   // overlap, bytes of the plane's own rows; no offset wraps, which the
   // launch checks) and are masked when published.
-  auto issue = [&](Stage& st, const Coords& c, int32_t tile) {
+  auto issue = [&](Stage& st, const Coords& c, int32_t tile) __attribute__((always_inline)) {
     const char* kp = static_cast<const char*>(p.k) + (c.b * p.sk[0] + c.h * p.sk[1]) * 2;
     const char* vp = static_cast<const char*>(p.v) + (c.b * p.sv[0] + c.h * p.sv[1]) * 2;
     const auto k_rsrc = plane_rsrc(kp, static_cast<uint32_t>(n_k - 1) * k_row_bytes + kD * 2);
@@ -226,7 +243,7 @@ rbf_tile_kernel(Problem p, int32_t q_blocks) {
       st.k[s] = load16_buf(k_rsrc, k_lane + row0 * k_row_bytes);
       st.v[s] = load16_buf(v_rsrc, v_lane + row0 * v_row_bytes);
     }
-    if (has_bias) {
+    if constexpr (kBias) {
       const char* bp = static_cast<const char*>(p.bias) + (c.b * p.sbb + c.h * p.sbh) * bias_esize;
       st.bias_misalign = base_misalign(bp);
 #pragma unroll
@@ -241,7 +258,7 @@ rbf_tile_kernel(Problem p, int32_t q_blocks) {
   // Writes a staged tile into LDS buffer `buf`: K and V rows, and per key
   // c_j = log2(e) bias_j - coef |k_j|^2 / 2 (-inf past Nk).  A fast pass
   // stores bf16 values as fp16 (to nearest).
-  auto publish = [&](const Stage& st, int32_t tile, int buf, float coef, auto kind_c) {
+  auto publish = [&](const Stage& st, int32_t tile, int buf, float coef, auto kind_c) __attribute__((always_inline)) {
     constexpr bool kFast = decltype(kind_c)::value == kPassFast;
     constexpr bool kToF16 = kFast && kBf16;
     const int32_t j0 = tile * kKeys;
@@ -280,15 +297,20 @@ rbf_tile_kernel(Problem p, int32_t q_blocks) {
         *reinterpret_cast<uint4*>(vl + key * G::kVStride + d0) = vw;
         // |k|^2 over the chunks of the row (kChunks adjacent lanes).
         const float sq = reduce_low<kChunks>(dot_chunk<T>(st.k[s], st.k[s], 0.f), OpSum());
-        if (slot % kChunks == 0) {
-          float bias = 0.f;
-          if (has_bias) {
-            const uint32_t j = static_cast<uint32_t>(min(j0 + key, n_k - 1));
-            const uint32_t bytes = j * static_cast<uint32_t>(p.sbn) * bias_esize + st.bias_misalign;
-            bias = decode_raw_scalar(RawScalar{st.bias[s], (bytes & 2u) * 8u}, p.bias_dtype) * kLog2e;
-          }
-          cl[key] = j0 + key < n_k ? fmaf(-0.5f * coef, sq, bias) : -INFINITY;
+        float bias = 0.f;
+        if constexpr (kBias) {
+          const uint32_t j = static_cast<uint32_t>(min(j0 + key, n_k - 1));
+          const uint32_t bytes = j * static_cast<uint32_t>(p.sbn) * bias_esize + st.bias_misalign;
+          bias = decode_raw_scalar(RawScalar{st.bias[s], (bytes & 2u) * 8u}, p.bias_dtype) * kLog2e;
+          // A masked key whose K row has a finite norm and whose V row is
+          // finite weighs exactly 0 and adds exact zeros.
+          const bool unmasked = j0 + key < n_k && !(bias == -INFINITY && __builtin_isfinite(sq));
+          any_live = any_live || unmasked;
+          const bool counts = unmasked || (j0 + key < n_k && !finite_chunk<T>(st.v[s]));
+          const uint64_t pieces = __builtin_amdgcn_ballot_w64(counts);
+          if (lane == 0) piece_live[buf][s * kWaves + wave] = pieces != 0;
         }
+        if (slot % kChunks == 0) cl[key] = j0 + key < n_k ? fmaf(-0.5f * coef, sq, bias) : -INFINITY;
       }
     }
   };
@@ -307,14 +329,35 @@ rbf_tile_kernel(Problem p, int32_t q_blocks) {
   // the diagonal holds every query's sum of squared weights.
   f32x4 wsq[kCB];
 
-  // Reduces tile `buf` for the wave's 16 * kCB queries.
-  auto compute = [&](int buf, float coef, auto kind_c) {
+  // Whether key pair kp of tile `tile` in buffer `buf` has a key that counts
+  // (wave-uniform): a piece is 64 / kChunks keys, a pair kChunks / 2 pieces.
+  auto pair_live = [&](int buf, int32_t tile, int kp) __attribute__((always_inline)) {
+    if (tile * kKeys + 32 * kp >= n_k) return false;
+    const uint8_t* at = &piece_live[buf][kp * (kChunks / 2)];
+    uint32_t any;
+    if constexpr (kChunks == 4) {
+      any = *reinterpret_cast<const uint16_t*>(at);
+    } else if constexpr (kChunks == 8) {
+      any = *reinterpret_cast<const uint32_t*>(at);
+    } else {
+      any = reinterpret_cast<const uint32_t*>(at)[0] | reinterpret_cast<const uint32_t*>(at)[1];
+    }
+    return __builtin_amdgcn_readfirstlane(any) != 0;
+  };
+
+  // Reduces tile `tile` (in buffer `buf`) for the wave's 16 * kCB queries.
+  auto compute = [&](int buf, int32_t tile, float coef, auto kind_c) __attribute__((always_inline)) {
     constexpr int kind = decltype(kind_c)::value;
     const T* kl = reinterpret_cast<const T*>(lds + buf * G::kBufBytes);
     const T* vl = reinterpret_cast<const T*>(lds + buf * G::kBufBytes + G::kKBytes);
     const float* cl = reinterpret_cast<const float*>(lds + buf * G::kBufBytes + G::kKBytes + G::kVBytes);
 #pragma unroll
     for (int kp = 0; kp < G::kPairs; ++kp) {
+      // Key pairs without a key that counts are skipped (the unshifted passes
+      // have no bias).
+      if constexpr (kBias) {
+        if (!pair_live(buf, tile, kp)) continue;
+      }
       // S^T for key blocks 2kp, 2kp + 1 and both query blocks.
       f32x4 s[kCB][2];
 #pragma unroll
@@ -438,7 +481,7 @@ rbf_tile_kernel(Problem p, int32_t q_blocks) {
   // the root of the key count), 2^-25 per key and for the values, against
   // `slack` times the allowance; also a weight sum (scaled to n_k keys) below
   // kFastSum / slack, or a non-finite output.
-  auto fast_misses = [&](float v_max, float seen, float slack) {
+  auto fast_misses = [&](float v_max, float seen, float slack) __attribute__((always_inline)) {
     const float grow = static_cast<float>(n_k) / seen;
     bool miss = false;
 #pragma unroll
@@ -471,9 +514,20 @@ rbf_tile_kernel(Problem p, int32_t q_blocks) {
   // contract by more than twice: the split pass then runs instead.  That is
   // a prediction, not the test: a fast pass that runs to the end is kept
   // only if its final sums pass it.
+  // Each query's maximum over its four lanes; 0 where it has no live key (the
+  // row then ends as NaN, or the range check sends the item on).
+  auto settle_max = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int cb = 0; cb < kCB; ++cb) {
+      const float m = allreduce_bit32(allreduce_bit16(row_max[cb], OpMax()), OpMax());
+      row_max[cb] = m == -INFINITY ? 0.f : m;
+    }
+  };
   Stage st;
   int32_t parity = 0;
-  auto run_pass = [&](const Coords& c, float coef, auto kind_c) {
+  // A shifted pass with `guess` takes the first tile's largest logits as its
+  // shift.
+  auto run_pass = [&](const Coords& c, float coef, bool active, bool guess, auto kind_c) __attribute__((always_inline)) {
     constexpr bool kFast = decltype(kind_c)::value == kPassFast;
     if constexpr (decltype(kind_c)::value != kPassMax) {
 #pragma unroll
@@ -495,7 +549,19 @@ rbf_tile_kernel(Problem p, int32_t q_blocks) {
     if (tiles > 1) issue(st, c, 1);
     const int32_t probe = tiles / 8;  // tiles reduced when the fast pass checks its course
     for (int32_t t = 0; t < tiles; ++t) {
-      compute(t & 1, coef, kind_c);
+      if constexpr (kBias) {
+        if (active) {
+          if constexpr (decltype(kind_c)::value == kPassShifted) {
+            if (guess && t == 0) {
+              compute(0, 0, coef, PassKind<kPassMax>{});
+              settle_max();
+            }
+          }
+          compute(t & 1, t, coef, kind_c);
+        }
+      } else {
+        compute(t & 1, t, coef, kind_c);
+      }
       if (t + 1 < tiles) publish(st, t + 1, (t + 1) & 1, coef, kind_c);
       if constexpr (kFast) {
         // After the staging registers are written out: no loads in flight.
@@ -523,7 +589,11 @@ rbf_tile_kernel(Problem p, int32_t q_blocks) {
       exact_flag[parity] = 0;
       split_flag[parity] = 0;
       abort_flag[parity] = 0;
+      live_flag[parity] = 0;
     }
+    // Waves whose queries are all past Nq stage tiles and keep the barriers.
+    const bool active = c.qb * G::kQRows + wave * kCB * 16 < n_q;
+    any_live = false;
     const float coef = 2.f * kLog2e * load_any(p.scale, c.b * p.ssb + c.h * p.ssh, p.scale_dtype);
     // Query rows of this wave: item rows (wave * kCB + cb) * 16 + col (rows
     // past Nq read row Nq - 1 and are not stored).
@@ -542,49 +612,72 @@ rbf_tile_kernel(Problem p, int32_t q_blocks) {
         q_half[cb] = f32x4{h, h, h, h};
       }
     }
-    // The single pass needs x <= 0: no bias and gamma >= 0.
-    bool exact = has_bias || !(coef >= 0.f);
-    bool split = true;
-    if (!exact && n_k >= kFastKeys && !(p.flags & VECTRA_FLAG_SPLIT_WEIGHTS)) {
-      // The fast result stands if the whole pass ran and its final sums pass
-      // the check anywhere in the workgroup: every weight sum at least
-      // kFastSum, every output finite and within the contract by its bound.
-      if (run_pass(c, coef, PassKind<kPassFast>{})) {
-        // The workgroup's max |v| (every wave staged a share of every tile).
-        const float m = kBf16 ? vmax : fmaxf(static_cast<float>(vmax16.x), static_cast<float>(vmax16.y));
-        const float mw = reduce_wave(m, OpMax());
-        if (lane == 0) vmax_wave[parity][wave] = mw;
-        __syncthreads();
-        float v_max = vmax_wave[parity][0];
+    // A weight sum outside the accurate range (or NaN, or a value that is not
+    // finite) anywhere in the workgroup sends the item to the exact passes.
+    auto redo_item = [&](bool out_of_range) __attribute__((always_inline)) {
+      if (active && __builtin_amdgcn_ballot_w64(out_of_range) && lane == 0) exact_flag[parity] = 1;
+      __syncthreads();
+      return exact_flag[parity] != 0;
+    };
+    bool exact = true;   // passes are left to do
+    bool guess = false;  // ... the next one shifted by the first tile's largest logits
+    if constexpr (kBias) {
+      guess = true;
+    } else if (coef >= 0.f) {  // the unshifted passes need x <= 0
+      bool split = true;
+      if (n_k >= kFastKeys && !(p.flags & VECTRA_FLAG_SPLIT_WEIGHTS)) {
+        // The fast result stands if the whole pass ran and its final sums pass
+        // the check anywhere in the workgroup: every weight sum at least
+        // kFastSum, every output finite and within the contract by its bound.
+        if (run_pass(c, coef, active, false, PassKind<kPassFast>{})) {
+          // The workgroup's max |v| (every wave staged a share of every tile).
+          const float m = kBf16 ? vmax : fmaxf(static_cast<float>(vmax16.x), static_cast<float>(vmax16.y));
+          const float mw = reduce_wave(m, OpMax());
+          if (lane == 0) vmax_wave[parity][wave] = mw;
+          __syncthreads();
+          float v_max = vmax_wave[parity][0];
 #pragma unroll
-        for (int w = 1; w < kWaves; ++w) v_max = fmaxf(v_max, vmax_wave[parity][w]);
-        const bool redo = fast_misses(v_max, static_cast<float>(n_k), 1.f);
-        if (__builtin_amdgcn_ballot_w64(redo) && lane == 0) split_flag[parity] = 1;
-        __syncthreads();
-        split = split_flag[parity] != 0;
+          for (int w = 1; w < kWaves; ++w) v_max = fmaxf(v_max, vmax_wave[parity][w]);
+          const bool redo = fast_misses(v_max, static_cast<float>(n_k), 1.f);
+          if (__builtin_amdgcn_ballot_w64(redo) && lane == 0) split_flag[parity] = 1;
+          __syncthreads();
+          split = split_flag[parity] != 0;
+        }
+      }
+      exact = false;
+      if (split) {
+        run_pass(c, coef, active, false, PassKind<kPassSum>{});
+        bool low = false;
+#pragma unroll
+        for (int cb = 0; cb < kCB; ++cb) low = low || !(total[cb][0] >= kSumLo);
+        exact = redo_item(low);
       }
     }
-    if (!exact && split) {
-      run_pass(c, coef, PassKind<kPassSum>{});
-      // A weight sum below the accurate range (or NaN) anywhere in the
-      // workgroup sends the item to the exact passes.
-      bool low = false;
-#pragma unroll
-      for (int cb = 0; cb < kCB; ++cb) low = low || !(total[cb][0] >= kSumLo);
-      if (__builtin_amdgcn_ballot_w64(low) && lane == 0) exact_flag[parity] = 1;
-      __syncthreads();
-      exact = exact_flag[parity] != 0;
-    }
-    if (exact) {
+    // With a bias, one pass shifted by the first tile's largest logits; where
+    // that leaves the range, and for gamma < 0, the exact passes: each query's
+    // largest logit, then the pass shifted by it.
+    while (exact) {
 #pragma unroll
       for (int cb = 0; cb < kCB; ++cb) row_max[cb] = -INFINITY;
-      run_pass(c, coef, PassKind<kPassMax>{});
+      if (!guess) {
+        run_pass(c, coef, active, false, PassKind<kPassMax>{});
+        settle_max();
+      }
+      run_pass(c, coef, active, guess, PassKind<kPassShifted>{});
+      if (!guess) break;
+      bool off = false;
 #pragma unroll
       for (int cb = 0; cb < kCB; ++cb) {
-        const float m = allreduce_bit32(allreduce_bit16(row_max[cb], OpMax()), OpMax());
-        row_max[cb] = m == -INFINITY ? 0.f : m;  // every key masked: the row ends as NaN
+        off = off || !(total[cb][0] >= kSumLo && total[cb][0] <= kSumHi);
+#pragma unroll
+        for (int u = 0; u < kDTiles; ++u)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) off = off || !__builtin_isfinite(acc[cb][u][r]);
       }
-      run_pass(c, coef, PassKind<kPassShifted>{});
+      if (__builtin_amdgcn_ballot_w64(any_live) && lane == 0) live_flag[parity] = 1;
+      // Without a live key every sum is 0 and every row NaN already.
+      exact = redo_item(off) && live_flag[parity] != 0;
+      guess = false;
     }
 
     // Store: every row of the ones product holds the query's weight sum; a
@@ -628,14 +721,14 @@ rbf_tile_kernel(Problem p, int32_t q_blocks) {
 
 // ------------------------------------------------------------------- host
 
-template <typename T, typename OutT, int kD, int kKeys, int kWaves, int kCB>
+template <typename T, typename OutT, int kD, int kKeys, int kWaves, int kCB, bool kBias>
 int tile_resident_blocks() {
   static std::atomic<int> cached{0};
   int n = cached.load(std::memory_order_relaxed);
   if (n == 0) {
     using G = TileGeo<T, kD, kKeys, kWaves, kCB>;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &n, reinterpret_cast<const void*>(&rbf_tile_kernel<T, OutT, kD, kKeys, kWaves, kCB>), 64 * kWaves,
+            &n, reinterpret_cast<const void*>(&rbf_tile_kernel<T, OutT, kD, kKeys, kWaves, kCB, kBias>), 64 * kWaves,
             2 * G::kBufBytes) != hipSuccess ||
         n < 1)
       n = 1;
@@ -644,12 +737,12 @@ int tile_resident_blocks() {
   return n;
 }
 
-template <typename T, typename OutT, int kD, int kKeys, int kWaves, int kCB>
-hipError_t launch_tile_k(Problem& p, hipStream_t s) {
+template <typename T, typename OutT, int kD, int kKeys, int kWaves, int kCB, bool kBias>
+hipError_t launch_tile_bias(Problem& p, hipStream_t s) {
   using G = TileGeo<T, kD, kKeys, kWaves, kCB>;
   const int32_t q_blocks = static_cast<int32_t>((p.Nq + G::kQRows - 1) / G::kQRows);
   const int64_t items = p.B * p.H * q_blocks;
-  int64_t blocks = static_cast<int64_t>(tile_resident_blocks<T, OutT, kD, kKeys, kWaves, kCB>()) *
+  int64_t blocks = static_cast<int64_t>(tile_resident_blocks<T, OutT, kD, kKeys, kWaves, kCB, kBias>()) *
                    (p.compute_units > 0 ? p.compute_units : 1);
   if (blocks > items) blocks = items;
   if (blocks >= 8) blocks -= blocks % 8;  // whole XCD rounds (see the kernel)
@@ -658,16 +751,44 @@ hipError_t launch_tile_k(Problem& p, hipStream_t s) {
   make_fast_div(q_blocks, &k.nq_mul, &k.nq_shift);
   int32_t qb = q_blocks;
   void* args[] = {&k, &qb};
-  return hipLaunchKernel(reinterpret_cast<const void*>(&rbf_tile_kernel<T, OutT, kD, kKeys, kWaves, kCB>),
+  return hipLaunchKernel(reinterpret_cast<const void*>(&rbf_tile_kernel<T, OutT, kD, kKeys, kWaves, kCB, kBias>),
                          dim3(static_cast<unsigned>(blocks)), dim3(64 * kWaves), args, 2 * G::kBufBytes, s);
+}
+
+template <typename T, typename OutT, int kD, int kKeys, int kWaves, int kCB>
+hipError_t launch_tile_k(Problem& p, hipStream_t s) {
+  return p.bias != nullptr ? launch_tile_bias<T, OutT, kD, kKeys, kWaves, kCB, true>(p, s)
+                           : launch_tile_bias<T, OutT, kD, kKeys, kWaves, kCB, false>(p, s);
 }
 
 template <typename T, typename OutT>
 hipError_t launch_tile_t(Problem& p, hipStream_t s) {
+  // Planes whose keys fit LDS are staged once for all their queries.
+  if (p.Nk <= kBlockMaxKeys) {
+    if (p.D == 32 && block_lds_bytes<32>(p.Nk) <= kBlockLdsBytes) return launch_block_d<T, OutT, 32>(p, s);
+    if (p.D == 64 && block_lds_bytes<64>(p.Nk) <= kBlockLdsBytes) return launch_block_d<T, OutT, 64>(p, s);
+    if (p.D == 128 && block_lds_bytes<128>(p.Nk) <= kBlockLdsBytes) return launch_block_d<T, OutT, 128>(p, s);
+  }
+  // Query blocks per wave: four share a tile's staging and operand reads best
+  // (two for 128-dim heads, by registers), as long as the work items fill the
+  // chip's resident workgroups; else two, else one.  Measured with 1 / 2 / 4,
+  // 64 dims, us: 256 planes of 4096 x 4096 2182 / 1547 / 1308, 64 of 2048 x 2048
+  // 274 / 220 / 194, 32 of 3000 x 3000 270 / 206 / 278, 8 of 4096 x 4096 113 /
+  // 121 / 167, 32 of 700 x 700 with a mask 24.8 / 30.0 / 38.2.
+  const int64_t planes = p.B * p.H, units = p.compute_units > 0 ? p.compute_units : 1;
+  auto items = [&](int64_t cb) { return planes * ((p.Nq + 64 * cb - 1) / (64 * cb)); };
   switch (p.D) {
-    case 32: return launch_tile_k<T, OutT, 32, 64, 4, 2>(p, s);
-    case 64: return launch_tile_k<T, OutT, 64, 64, 4, 4>(p, s);
-    case 128: return launch_tile_k<T, OutT, 128, 32, 4, 2>(p, s);
+    case 32:
+      if (items(4) >= 2 * units) return launch_tile_k<T, OutT, 32, 64, 4, 4>(p, s);
+      if (items(2) > units) return launch_tile_k<T, OutT, 32, 64, 4, 2>(p, s);
+      return launch_tile_k<T, OutT, 32, 64, 4, 1>(p, s);
+    case 64:
+      if (items(4) >= 2 * units) return launch_tile_k<T, OutT, 64, 64, 4, 4>(p, s);
+      if (items(2) >= 2 * units) return launch_tile_k<T, OutT, 64, 64, 4, 2>(p, s);
+      return launch_tile_k<T, OutT, 64, 64, 4, 1>(p, s);
+    case 128:
+      if (items(2) > units) return launch_tile_k<T, OutT, 128, 32, 4, 2>(p, s);
+      return launch_tile_k<T, OutT, 128, 32, 4, 1>(p, s);
     default: return hipErrorInvalidValue;
   }
 }
