@@ -523,6 +523,102 @@ __global__ __launch_bounds__(kAdcThreads) void pq_adc_vec_kernel(PqAdc p) {
   }
 }
 
+// Several queries over short codes (at most 32 bytes on 8- or 16-byte
+// boundaries): a workgroup holds the tables of kQ queries interleaved, entry
+// (s, c) of all of them in one 4 kQ-byte word, so one LDS read and one code
+// serve kQ distances.  Bound: the lookups (64 lanes gather from random banks)
+// and, with four queries, nearly HBM.  Loads as in pq_adc_vec_kernel, each
+// distance's sums adc_sum's.  Measured, one workgroup set per query before and
+// this, us: 8 queries x 1M 16-byte codes 29.8 and 14.5 (48 MB: 7.5 at a plain
+// read's rate), 4 x 2M 8-byte codes 23.5 and 10.7, 32 x 500k 8-byte codes 79.5
+// and 14.9, 16 x 200k 32-byte codes 40.1 and 14.1; two queries per workgroup
+// 15.1, 10.7, 16.4 and 14.9.
+// kWords: 32-bit words of a code's loads; kM: sub-spaces when known, else 0.
+constexpr int kAdcMultiThreads = 1024;
+
+template <int kQ, int kWords, int kM, bool kIds>
+__global__ __launch_bounds__(kAdcMultiThreads) void pq_adc_multi_kernel(PqAdc p, int64_t num_queries) {
+  extern __shared__ __align__(16) float multi_lds[];  // [subspaces * 256][kQ]
+  typedef float Entries __attribute__((ext_vector_type(kQ)));
+  Entries* table = reinterpret_cast<Entries*>(multi_lds);
+  const int m = kM > 0 ? kM : p.subspaces;
+  const int64_t q0 = static_cast<int64_t>(blockIdx.y) * kQ;
+  const int nq = static_cast<int>(num_queries - q0 < kQ ? num_queries - q0 : kQ);
+  const int64_t stride = static_cast<int64_t>(gridDim.x) * kAdcMultiThreads;
+  const int64_t last = p.num_cand - 1;
+  auto load = [&](int64_t cand, bool& valid, uint32_t (&code)[kWords]) {
+    const int64_t c = cand < last ? cand : last;
+    int64_t index = c;
+    valid = cand <= last;
+    if constexpr (kIds) {
+      const uint32_t id = p.ids[c];
+      valid = valid && static_cast<int64_t>(id) < p.num_codes;
+      index = valid ? static_cast<int64_t>(id) : 0;
+    }
+    const uint8_t* at = p.codes + index * p.code_stride;
+    if constexpr (kWords == 2) {
+      const uint2 x = *reinterpret_cast<const uint2*>(at);
+      code[0] = x.x;
+      code[1] = x.y;
+    } else {
+#pragma unroll
+      for (int k = 0; k < kWords / 4; ++k) {
+        const uint4 x = *reinterpret_cast<const uint4*>(at + 16 * k);
+        code[4 * k] = x.x;
+        code[4 * k + 1] = x.y;
+        code[4 * k + 2] = x.z;
+        code[4 * k + 3] = x.w;
+      }
+    }
+  };
+  int64_t cand = static_cast<int64_t>(blockIdx.x) * kAdcMultiThreads + threadIdx.x;
+  bool valid_a, valid_b;
+  uint32_t code_a[kWords], code_b[kWords];
+  load(cand, valid_a, code_a);
+  for (int i = static_cast<int>(threadIdx.x); i < m * VECTRA_PQ_CENTROIDS; i += kAdcMultiThreads) {
+    Entries e;
+#pragma unroll
+    for (int j = 0; j < kQ; ++j) e[j] = p.tables[(q0 + (j < nq ? j : nq - 1)) * p.table_stride + i];
+    table[i] = e;
+  }
+  __syncthreads();
+  auto emit = [&](int64_t at, bool valid, const uint32_t (&code)[kWords]) {
+    auto entry = [&](int s, uint32_t c) { return table[s * VECTRA_PQ_CENTROIDS + static_cast<int>(c)]; };
+    Entries l0 = 0.f, l1 = 0.f, l2 = 0.f, l3 = 0.f;
+#pragma unroll
+    for (int k = 0; k < kWords; ++k) {
+      if (4 * k + 4 <= m) {
+        const uint32_t w = code[k];
+        l0 = l0 + entry(4 * k, w & 0xffu);
+        l1 = l1 + entry(4 * k + 1, (w >> 8) & 0xffu);
+        l2 = l2 + entry(4 * k + 2, (w >> 16) & 0xffu);
+        l3 = l3 + entry(4 * k + 3, w >> 24);
+      }
+    }
+    Entries sum = (l0 + l1) + (l2 + l3);
+    if constexpr (kM == 0) {
+      const int full = m & ~3;
+      uint32_t rest = 0;
+#pragma unroll
+      for (int k = 0; k < kWords; ++k)
+        if (k == full / 4) rest = code[k];
+#pragma unroll
+      for (int r = 0; r < 3; ++r)
+        if (full + r < m) sum = sum + entry(full + r, (rest >> (8 * r)) & 0xffu);
+    }
+#pragma unroll
+    for (int j = 0; j < kQ; ++j)
+      if (at <= last && j < nq)
+        __builtin_nontemporal_store(valid ? sum[j] : NAN, &p.out[(q0 + j) * p.out_stride + at]);
+  };
+  for (; cand <= last; cand += 2 * stride) {
+    load(cand + stride, valid_b, code_b);
+    emit(cand, valid_a, code_a);
+    load(cand + 2 * stride, valid_a, code_a);
+    emit(cand + stride, valid_b, code_b);
+  }
+}
+
 unsigned blocks_for(int64_t items, int per_block, int64_t cap = kMaxBlocksX) {
   int64_t blocks = (items + per_block - 1) / per_block;
   if (blocks > cap) blocks = cap;
@@ -1105,6 +1201,39 @@ extern "C" int vectra_pq_distance_tables(const vectra_pq_table_args* a, hipStrea
                                   dim3(kThreads), args, 0, stream));
 }
 
+namespace {
+
+template <int kQ, int kWords, int kM>
+int launch_adc_multi_k(PqAdc& p, int64_t queries, hipStream_t stream) {
+  void* args[] = {&p, &queries};
+  const int64_t y = (queries + kQ - 1) / kQ;
+  const size_t lds = static_cast<size_t>(p.subspaces) * VECTRA_PQ_CENTROIDS * kQ * sizeof(float);
+  const int64_t per_cu = lds <= 80 * 1024 ? 2 : 1;
+  int64_t x = (256 * per_cu + y - 1) / y;
+  const dim3 grid(blocks_for(p.num_cand, kAdcMultiThreads, x < 1 ? 1 : x), static_cast<unsigned>(y));
+  const void* kernel = p.ids != nullptr ? reinterpret_cast<const void*>(&pq_adc_multi_kernel<kQ, kWords, kM, true>)
+                                        : reinterpret_cast<const void*>(&pq_adc_multi_kernel<kQ, kWords, kM, false>);
+  return launched(hipLaunchKernel(kernel, grid, dim3(kAdcMultiThreads), args, lds, stream));
+}
+
+// kQ is 1 for codes of at most 8 bytes only.
+template <int kQ>
+int launch_adc_multi(PqAdc& p, int64_t queries, hipStream_t stream) {
+  const int m = p.subspaces;
+  if (m == 8) return launch_adc_multi_k<kQ, 2, 8>(p, queries, stream);
+  if (m < 8 && p.code_stride % 8 == 0 && reinterpret_cast<uintptr_t>(p.codes) % 8 == 0)
+    return launch_adc_multi_k<kQ, 2, 0>(p, queries, stream);
+  if constexpr (kQ > 1) {
+    if (m == 16) return launch_adc_multi_k<kQ, 4, 16>(p, queries, stream);
+    if (m < 16) return launch_adc_multi_k<kQ, 4, 0>(p, queries, stream);
+    if (m == 32) return launch_adc_multi_k<kQ, 8, 32>(p, queries, stream);
+    return launch_adc_multi_k<kQ, 8, 0>(p, queries, stream);
+  }
+  return VECTRA_SCAN_LAUNCH_FAILED;  // not reached
+}
+
+}  // namespace
+
 extern "C" int vectra_scan_pq_adc(const vectra_pq_adc_args* a, hipStream_t stream) {
   if (a == nullptr) return VECTRA_SCAN_INVALID_ARGUMENT;
   if (a->subspaces < 1 || a->subspaces > VECTRA_PQ_CENTROIDS || a->num_queries < 0 || a->num_codes < 0 ||
@@ -1138,6 +1267,13 @@ extern "C" int vectra_scan_pq_adc(const vectra_pq_adc_args* a, hipStream_t strea
   void* args[] = {&p};
   const dim3 grid(blocks_for(cand, kThreads, kScanBlocks), static_cast<unsigned>(a->num_queries));
   const bool vec16 = a->code_stride % 16 == 0 && reinterpret_cast<uintptr_t>(a->codes) % 16 == 0;
+  // Two queries or more share each code and lookup; so do one query's codes of
+  // at most 8 bytes, which the single-query kernel does not take.
+  const bool vec8 = a->subspaces <= 8 && a->code_stride % 8 == 0 && reinterpret_cast<uintptr_t>(a->codes) % 8 == 0;
+  if (a->num_codes > 0 && (vec8 || (vec16 && a->subspaces <= 32 && a->num_queries > 1))) {
+    if (a->num_queries == 1) return launch_adc_multi<1>(p, 1, stream);
+    return a->num_queries == 2 ? launch_adc_multi<2>(p, 2, stream) : launch_adc_multi<4>(p, a->num_queries, stream);
+  }
   if (vec16 && a->subspaces <= 32 && a->num_codes > 0) {
     const size_t lds = static_cast<size_t>(entries) * sizeof(float);
     const bool ids = a->ids != nullptr;
