@@ -1387,6 +1387,16 @@ int launch_top_k(int64_t queries, TopK& p, hipStream_t stream) {
   void* args[] = {&p};
   const bool ids = p.ids != nullptr;
   const bool d128 = p.dim == 128;
+  // Ranges of the split form: 16 waves load a long range four times as wide
+  // and sort a large selection on four times the threads; a short one is
+  // over sooner on 4 waves.  Measured, 4 and 16 waves, us: 1 query x 200,000 x
+  // 128, k = 10 (3,125 candidates a range) 79 and 73, x 300,000 x 64 206 and 65,
+  // 3 x 100,000 x 100 119 and 52, 2 x 20,000 x 128, k = 100 (1,250) 98 and 65,
+  // 3 x 8,000, k = 100 (500) 64 and 53; 1 x 100,000, k = 10 (1,563) 44 and 46,
+  // x 50,000 28 and 33.
+  if (p.splits > 1 && (p.split_len >= 2048 || (p.k > kWaveLanes && p.split_len >= 400)))
+    return launched(hipLaunchKernel(d128 ? top_k_kernel<1024, 4, 1, 128>(ids) : top_k_kernel<1024, 6, 1, 0>(ids),
+                                    dim3(static_cast<unsigned>(queries * p.splits)), dim3(1024), args, 0, stream));
   if (p.splits > 1)
     return launched(hipLaunchKernel(d128 ? top_k_kernel<256, 4, 1, 128>(ids) : top_k_kernel<256, 4, 1, 0>(ids),
                                     dim3(static_cast<unsigned>(queries * p.splits)), dim3(256), args, 0, stream));
