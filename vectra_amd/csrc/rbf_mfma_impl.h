@@ -105,7 +105,8 @@ struct MfmaOffsets {
   uint32_t bias[Stage::kBSlots];  // elements
 };
 
-template <typename T, typename OutT, int kD, int kKeys, int kWaves>
+// kSkip: fp32 with a bias.
+template <typename T, typename OutT, int kD, int kKeys, int kWaves, bool kSkip>
 __global__ __launch_bounds__(64 * kWaves) void rbf_mfma_kernel(Problem p, int32_t q_blocks) {
   using Geo = MfmaTile<T, kD, kKeys>;
   using Stage = MfmaStage<T, kD, kKeys, kWaves>;
@@ -126,6 +127,14 @@ __global__ __launch_bounds__(64 * kWaves) void rbf_mfma_kernel(Problem p, int32_
   T* v_lds = reinterpret_cast<T*>(lds + Geo::kKBytes);
   float* kn_lds = reinterpret_cast<float*>(lds + Geo::kKBytes + Geo::kVBytes);
   float* bias_lds = kn_lds + kKeys;
+  // fp32 with a bias, bit t of live_blocks[n & 1]: 16-key block t of the n-th
+  // tile holds a key that counts (not masked by a -inf bias, or with a K norm
+  // or V row that is not finite).  The products of the other blocks are
+  // skipped: their weights are exactly 0.  (260 planes of 291 x 291 x 64 with
+  // half the keys masked 117 -> 86 us; without a bias the marks cost 6%, so
+  // that kernel is built without them.)
+  static_assert(!kSkip || !kHalf, "a staging slot's keys lie in one block: fp32 rows");
+  __shared__ uint32_t live_blocks[2];
 
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
@@ -232,8 +241,12 @@ __global__ __launch_bounds__(64 * kWaves) void rbf_mfma_kernel(Problem p, int32_
   };
 
   // Copies a staged tile into LDS: K rows and -|k|^2 / 2, V, and biases.
-  auto publish = [&](const Stage& st, int32_t tile) {
+  auto publish = [&](const Stage& st, int32_t tile, int parity) {
     const int32_t j0 = tile * kKeys;
+    // Marks block `key` / 16 (one block for all keys of the wave's slot).
+    auto mark = [&](bool counts, int key) {
+      if (__builtin_amdgcn_ballot_w64(counts) != 0 && lane == 0) atomicOr(&live_blocks[parity], 1u << (key / 16));
+    };
 #pragma unroll
     for (int s = 0; s < Stage::kKSlots; ++s) {
       const int slot = tid + s * kThreads;
@@ -247,6 +260,7 @@ __global__ __launch_bounds__(64 * kWaves) void rbf_mfma_kernel(Problem p, int32_
       if (live) *reinterpret_cast<uint4*>(k_lds + key * Geo::kKStride + (slot % kDChunks) * kVec) = raw;
       const float sq = reduce_low<kDChunks>(dot_chunk<T>(raw, raw, 0.f), OpSum());
       if (live && slot % kDChunks == 0) kn_lds[key] = -0.5f * sq;
+      if constexpr (kSkip) mark(live && !__builtin_isfinite(sq), key);
     }
 #pragma unroll
     for (int s = 0; s < Stage::kVSlots; ++s) {
@@ -269,6 +283,10 @@ __global__ __launch_bounds__(64 * kWaves) void rbf_mfma_kernel(Problem p, int32_
           }
         } else {
           const uint4 r0 = j0 + row < n_k ? st.v[s][0] : make_uint4(0, 0, 0, 0);
+          if constexpr (kSkip)
+            mark(!(__builtin_isfinite(__uint_as_float(r0.x)) && __builtin_isfinite(__uint_as_float(r0.y)) &&
+                   __builtin_isfinite(__uint_as_float(r0.z)) && __builtin_isfinite(__uint_as_float(r0.w))),
+                 row);
           float* dst = reinterpret_cast<float*>(v_lds) + ((row >> 2) * kD + d0) * 4 + (row & 3);
           dst[0] = __uint_as_float(r0.x);
           dst[4] = __uint_as_float(r0.y);
@@ -291,6 +309,11 @@ __global__ __launch_bounds__(64 * kWaves) void rbf_mfma_kernel(Problem p, int32_
           }
         }
         bias_lds[key] = x;
+        if constexpr (kSkip) {
+          // 16 keys of a lane group each; lane 0 of a group marks its block.
+          const uint64_t keys = __builtin_amdgcn_ballot_w64(!(x == -INFINITY));
+          if (col == 0 && ((keys >> (16 * grp)) & 0xffffu) != 0) atomicOr(&live_blocks[parity], 1u << (key / 16));
+        }
       }
     }
   };
@@ -302,6 +325,9 @@ __global__ __launch_bounds__(64 * kWaves) void rbf_mfma_kernel(Problem p, int32_
   Stage st;
   int32_t item = static_cast<int32_t>(blockIdx.x), tile = 0;
   if (item >= items) return;  // before any barrier: the whole workgroup leaves
+  int parity = 0;  // of the tiles reduced so far
+  bool active = true;  // the wave has query rows
+  if (kSkip && tid < 2) live_blocks[tid] = 0u;
   issue(st, item, 0);
   while (true) {
     int32_t next_item = item, next_tile = tile + 1;
@@ -310,9 +336,10 @@ __global__ __launch_bounds__(64 * kWaves) void rbf_mfma_kernel(Problem p, int32_
       next_item += static_cast<int32_t>(gridDim.x);
     }
     __syncthreads();  // the previous tile is no longer read from LDS
-    publish(st, tile);
+    publish(st, tile, parity);
     if (tile == 0) {
       const Coords c = coords(item);
+      if constexpr (kSkip) active = (c.qb * kWaves + wave) * 16 < n_q;
       const bool q_live = (c.qb * kWaves + wave) * 16 + col < n_q;
       float q_norm = 0.f;
 #pragma unroll
@@ -332,11 +359,21 @@ __global__ __launch_bounds__(64 * kWaves) void rbf_mfma_kernel(Problem p, int32_
     const bool more = next_item < items;
     if (more) issue(st, next_item, next_tile);  // in flight while this tile is reduced
 
+    // Key blocks to reduce; the next tile's word is cleared for its publish.
+    uint32_t live = ~0u;
+    if constexpr (kSkip) {
+      live = active ? __builtin_amdgcn_readfirstlane(live_blocks[parity]) : 0u;
+      parity ^= 1;
+      if (tid == 0) live_blocks[parity] = 0u;
+    }
     // Logits (log2 units) of this lane's query against keys 16t + 4g + r.
     float logit[kNTiles][4];
     float tile_max = -INFINITY;
 #pragma unroll
     for (int t = 0; t < kNTiles; ++t) {
+      if constexpr (kSkip) {
+        if (!(live & (1u << t))) continue;
+      }
       const float4 kn = *reinterpret_cast<const float4*>(kn_lds + 16 * t + 4 * grp);
       f32x4 sc = f32x4{kn.x + q_half, kn.y + q_half, kn.z + q_half, kn.w + q_half};
       if constexpr (kHalf) {
@@ -423,6 +460,9 @@ __global__ __launch_bounds__(64 * kWaves) void rbf_mfma_kernel(Problem p, int32_
     } else {
 #pragma unroll
       for (int t = 0; t < kNTiles; ++t) {
+        if constexpr (kSkip) {
+          if (!(live & (1u << t))) continue;
+        }
         float w[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) w[r] = __builtin_amdgcn_exp2f(logit[t][r] - safe_max);
@@ -476,14 +516,14 @@ __global__ __launch_bounds__(64 * kWaves) void rbf_mfma_kernel(Problem p, int32_
 
 // Workgroups of one MFMA instantiation that fit on a compute unit at once
 // (registers and LDS), asked of the runtime once per process.
-template <typename T, typename OutT, int kD, int kKeys, int kWaves>
+template <typename T, typename OutT, int kD, int kKeys, int kWaves, bool kSkip>
 int mfma_resident_blocks() {
   static std::atomic<int> cached{0};
   int n = cached.load(std::memory_order_relaxed);
   if (n == 0) {
     using Geo = MfmaTile<T, kD, kKeys>;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &n, reinterpret_cast<const void*>(&rbf_mfma_kernel<T, OutT, kD, kKeys, kWaves>), 64 * kWaves,
+            &n, reinterpret_cast<const void*>(&rbf_mfma_kernel<T, OutT, kD, kKeys, kWaves, kSkip>), 64 * kWaves,
             Geo::kBytes) != hipSuccess ||
         n < 1)
       n = 1;
@@ -495,12 +535,12 @@ int mfma_resident_blocks() {
 // The grid is persistent: as many workgroups as are resident at once, each
 // looping over work items, so one item's loads overlap the previous one's
 // products.
-template <typename T, typename OutT, int kD, int kKeys, int kWaves>
-hipError_t launch_mfma_w(Problem& p, hipStream_t s) {
+template <typename T, typename OutT, int kD, int kKeys, int kWaves, bool kSkip>
+hipError_t launch_mfma_s(Problem& p, hipStream_t s) {
   using Geo = MfmaTile<T, kD, kKeys>;
   const int32_t q_blocks = static_cast<int32_t>((p.Nq + kWaves * 16 - 1) / (kWaves * 16));
   const int64_t items = p.B * p.H * q_blocks;
-  int64_t blocks = static_cast<int64_t>(mfma_resident_blocks<T, OutT, kD, kKeys, kWaves>()) *
+  int64_t blocks = static_cast<int64_t>(mfma_resident_blocks<T, OutT, kD, kKeys, kWaves, kSkip>()) *
                    (p.compute_units > 0 ? p.compute_units : 1);
   if (blocks > items) blocks = items;
   // Item indices (and item + grid size) stay below 2^31.
@@ -509,17 +549,33 @@ hipError_t launch_mfma_w(Problem& p, hipStream_t s) {
   make_fast_div(q_blocks, &k.nq_mul, &k.nq_shift);
   int32_t qb = q_blocks;
   void* args[] = {&k, &qb};
-  return hipLaunchKernel(reinterpret_cast<const void*>(&rbf_mfma_kernel<T, OutT, kD, kKeys, kWaves>),
+  return hipLaunchKernel(reinterpret_cast<const void*>(&rbf_mfma_kernel<T, OutT, kD, kKeys, kWaves, kSkip>),
                          dim3(static_cast<unsigned>(blocks)), dim3(64 * kWaves), args, Geo::kBytes, s);
+}
+
+template <typename T, typename OutT, int kD, int kKeys, int kWaves>
+hipError_t launch_mfma_w(Problem& p, hipStream_t s) {
+  if constexpr (sizeof(T) == 4) {
+    if (p.bias != nullptr) return launch_mfma_s<T, OutT, kD, kKeys, kWaves, true>(p, s);
+  }
+  return launch_mfma_s<T, OutT, kD, kKeys, kWaves, false>(p, s);
 }
 
 // Waves per workgroup: one per 16-row query tile of a plane, at least 4 (the
 // loaders' register staging of a tile is split over the workgroup) and at
-// most 8; 5 covers the 65-token comparable sets.
+// most 8; 5 covers the 65-token comparable sets.  fp32 with a bias takes 4
+// where 8 would leave CUs idle, and from 1.25 items of 8 waves per CU on
+// (finer ones balance ragged planes): 8 planes of 900 x 900 x 64 74 us with 8
+// waves and 58 with 4, 320 of 120 x 120 x 64 29 and 26, 180 of 431 x 431 x 32
+// 66 and 61; about one item of 8 waves per CU stays with 8 (64 planes of
+// 500 x 500 x 64 48 and 52).
 template <typename T, typename OutT, int kD, int kKeys>
 hipError_t launch_mfma_k(Problem& p, hipStream_t s) {
   const int64_t tiles = (p.Nq + 15) / 16;
-  if (tiles <= 4) return launch_mfma_w<T, OutT, kD, kKeys, 4>(p, s);
+  const int64_t units = p.compute_units > 0 ? p.compute_units : 1;
+  const int64_t items = p.B * p.H * ((tiles + 7) / 8);
+  const bool small = sizeof(T) == 4 && p.bias != nullptr && (4 * items < 3 * units || 4 * items >= 5 * units);
+  if (tiles <= 4 || small) return launch_mfma_w<T, OutT, kD, kKeys, 4>(p, s);
   if (tiles <= 5) return launch_mfma_w<T, OutT, kD, kKeys, 5>(p, s);
   return launch_mfma_w<T, OutT, kD, kKeys, 8>(p, s);
 }
