@@ -769,22 +769,25 @@ hipError_t launch_tile_t(Problem& p, hipStream_t s) {
     if (p.D == 64 && block_lds_bytes<64>(p.Nk) <= kBlockLdsBytes) return launch_block_d<T, OutT, 64>(p, s);
     if (p.D == 128 && block_lds_bytes<128>(p.Nk) <= kBlockLdsBytes) return launch_block_d<T, OutT, 128>(p, s);
   }
-  // Query blocks per wave: four share a tile's staging and operand reads best
-  // (two for 128-dim heads, by registers), as long as the work items fill the
-  // chip's resident workgroups; else two, else one.  Measured with 1 / 2 / 4,
-  // 64 dims, us: 256 planes of 4096 x 4096 2182 / 1547 / 1308, 64 of 2048 x 2048
-  // 274 / 220 / 194, 32 of 3000 x 3000 270 / 206 / 278, 8 of 4096 x 4096 113 /
-  // 121 / 167, 32 of 700 x 700 with a mask 24.8 / 30.0 / 38.2.
   const int64_t planes = p.B * p.H, units = p.compute_units > 0 ? p.compute_units : 1;
   auto items = [&](int64_t cb) { return planes * ((p.Nq + 64 * cb - 1) / (64 * cb)); };
+  auto rounds = [&](int64_t cb) { return (items(cb) + units - 1) / units; };
+  // Query blocks per wave: four share a tile's staging and operand reads best
+  // (two for 128-dim heads, by registers, and 32-dim ones, where an item of 256
+  // rows is taken again as a whole when one row's fp16 weights may miss the
+  // bound), but the launch lasts as long as the fullest CU's items.  An item of
+  // four blocks per wave costs 1 / 0.57 of one of two.  Measured with 4 / 2 / 1,
+  // 64 dims, us: 256 planes of 4096 x 4096 1308 / 1547 / 2182, 64 of 2048 x 2048
+  // 193 / 214 / 265, 152 of 731 x 2882 262 / 279 / 288, 520 of 256 x 4096 284 /
+  // 267 / 319, 32 of 3000 x 3000 264 / 199 / 252, 64 of 1000 x 4096 206 / 164 /
+  // 153; 32 dims: 152 of 731 x 2882 193 / 148 / 177, 400 of 700 x 2000 319 / 335 / 381.
   switch (p.D) {
     case 32:
-      if (items(4) >= 2 * units) return launch_tile_k<T, OutT, 32, 64, 4, 4>(p, s);
       if (items(2) > units) return launch_tile_k<T, OutT, 32, 64, 4, 2>(p, s);
       return launch_tile_k<T, OutT, 32, 64, 4, 1>(p, s);
     case 64:
-      if (items(4) >= 2 * units) return launch_tile_k<T, OutT, 64, 64, 4, 4>(p, s);
-      if (items(2) >= 2 * units) return launch_tile_k<T, OutT, 64, 64, 4, 2>(p, s);
+      if (rounds(4) >= 2 && 100 * rounds(4) < 57 * rounds(2)) return launch_tile_k<T, OutT, 64, 64, 4, 4>(p, s);
+      if (2 * items(2) >= 5 * units) return launch_tile_k<T, OutT, 64, 64, 4, 2>(p, s);
       return launch_tile_k<T, OutT, 64, 64, 4, 1>(p, s);
     case 128:
       if (items(2) > units) return launch_tile_k<T, OutT, 128, 32, 4, 2>(p, s);
