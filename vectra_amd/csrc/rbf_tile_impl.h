@@ -82,6 +82,7 @@
 #include "rbf_common.h"
 #include "rbf_kernels.h"
 #include "rbf_block_impl.h"
+#include "rbf_span_impl.h"
 #include "rbf_mfma_ops.h"
 #include "rbf_tile_ops.h"
 
@@ -772,6 +773,17 @@ hipError_t launch_tile_t(Problem& p, hipStream_t s) {
   const int64_t planes = p.B * p.H, units = p.compute_units > 0 ? p.compute_units : 1;
   auto items = [&](int64_t cb) { return planes * ((p.Nq + 64 * cb - 1) / (64 * cb)); };
   auto rounds = [&](int64_t cb) { return (items(cb) + units - 1) / units; };
+  // Few work items with a bias: the waves share out the keys instead of the
+  // queries, up to one 32-row item per CU (beyond, the streamed items gain more
+  // from the masked keys that they skip).  Without a bias the streamed kernel's
+  // fp16-weight pass makes the results of a long axis, which a plane's company
+  // must not change.  Measured, streamed and shared out, us: 176 items of 700
+  // masked keys 20 and 14, 352 of them 21 and 26.
+  if (p.bias != nullptr && planes * ((p.Nq + 31) / 32) <= units) {
+    if (p.D == 32) return launch_span<T, OutT, 32>(p, units, s);
+    if (p.D == 64) return launch_span<T, OutT, 64>(p, units, s);
+    if (p.D == 128) return launch_span<T, OutT, 128>(p, units, s);
+  }
   // Query blocks per wave: four share a tile's staging and operand reads best
   // (two for 128-dim heads, by registers, and 32-dim ones, where an item of 256
   // rows is taken again as a whole when one row's fp16 weights may miss the
