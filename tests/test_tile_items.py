@@ -38,3 +38,34 @@ def test_query_blocks_per_wave(planes, n_q, n_k, dim, masked):
         if masked:
             logits = logits + bias[plane, 0].double()
         torch.testing.assert_close(got[plane, 0].double(), torch.softmax(logits, -1) @ vd, rtol=1e-3, atol=1e-4)
+
+
+def _long_axis(n_q, n_k, dim):
+    """One batch entry on whose near rows one fp16 weight per key holds the
+    contract, with row n_q // 2 far from every key: its group of rows (256 for
+    64 dims, else 128) takes hi + lo weights as a whole."""
+    gen = torch.Generator(device='cuda').manual_seed(n_q + dim)
+    q, k = (0.5 * torch.randn(1, 1, n, dim, generator=gen, device='cuda') for n in (n_q, n_k))
+    v = 0.25 * torch.randn(1, 1, n_k, dim, generator=gen, device='cuda')
+    q[:, :, n_q // 2] += 4.0
+    return [t.bfloat16() for t in (q, k, v)] + [torch.full((1, 1, 1, 1), 0.64 / dim, device='cuda')]
+
+
+@pytest.mark.parametrize('n_q,n_k,dim', [(600, 2048, 64), (64, 1025, 64), (257, 1601, 64), (300, 2048, 32), (129, 1100, 32),
+                                         (200, 1100, 128)])
+@pytest.mark.parametrize('out_dtype', [torch.float32, torch.bfloat16], ids=str)
+def test_rows_do_not_depend_on_the_planes_beside_them(n_q, n_k, dim, out_dtype):
+    q, k, v, scale = _long_axis(n_q, n_k, dim)
+    alone = capi.forward(q, k, v, scale, out_dtype=out_dtype, variant='tile')
+    split = capi.forward(q, k, v, scale, out_dtype=torch.float32, variant='tile', split_weights=True)
+    assert not alone.isnan().any()
+    group = 256 if dim == 64 else 128
+    first = n_q // 2 // group * group
+    far = slice(first, min(first + group, n_q))
+    if out_dtype == torch.float32:
+        assert torch.equal(alone[:, :, far], split[:, :, far])
+        assert n_q <= group or not torch.equal(alone, split), 'no group kept its fp16 weights'
+    for planes in (3, 40, 150, 400, 700):
+        print(planes, n_q, n_k, dim, flush=True)
+        many = capi.forward(*(t.expand(planes, -1, -1, -1) for t in (q, k, v)), scale, out_dtype=out_dtype, variant='tile')
+        assert torch.equal(many, alone.expand_as(many)), planes

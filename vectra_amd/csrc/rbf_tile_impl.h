@@ -739,7 +739,7 @@ int tile_resident_blocks() {
 }
 
 template <typename T, typename OutT, int kD, int kKeys, int kWaves, int kCB, bool kBias>
-hipError_t launch_tile_bias(Problem& p, hipStream_t s) {
+hipError_t launch_tile_k(Problem& p, hipStream_t s) {
   using G = TileGeo<T, kD, kKeys, kWaves, kCB>;
   const int32_t q_blocks = static_cast<int32_t>((p.Nq + G::kQRows - 1) / G::kQRows);
   const int64_t items = p.B * p.H * q_blocks;
@@ -756,12 +756,6 @@ hipError_t launch_tile_bias(Problem& p, hipStream_t s) {
                          dim3(static_cast<unsigned>(blocks)), dim3(64 * kWaves), args, 2 * G::kBufBytes, s);
 }
 
-template <typename T, typename OutT, int kD, int kKeys, int kWaves, int kCB>
-hipError_t launch_tile_k(Problem& p, hipStream_t s) {
-  return p.bias != nullptr ? launch_tile_bias<T, OutT, kD, kKeys, kWaves, kCB, true>(p, s)
-                           : launch_tile_bias<T, OutT, kD, kKeys, kWaves, kCB, false>(p, s);
-}
-
 template <typename T, typename OutT>
 hipError_t launch_tile_t(Problem& p, hipStream_t s) {
   // Planes whose keys fit LDS are staged once for all their queries.
@@ -773,39 +767,49 @@ hipError_t launch_tile_t(Problem& p, hipStream_t s) {
   const int64_t planes = p.B * p.H, units = p.compute_units > 0 ? p.compute_units : 1;
   auto items = [&](int64_t cb) { return planes * ((p.Nq + 64 * cb - 1) / (64 * cb)); };
   auto rounds = [&](int64_t cb) { return (items(cb) + units - 1) / units; };
-  // Few work items with a bias: the waves share out the keys instead of the
-  // queries, up to one 32-row item per CU (beyond, the streamed items gain more
-  // from the masked keys that they skip).  Without a bias the streamed kernel's
-  // fp16-weight pass makes the results of a long axis, which a plane's company
-  // must not change.  Measured, streamed and shared out, us: 176 items of 700
-  // masked keys 20 and 14, 352 of them 21 and 26.
-  if (p.bias != nullptr && planes * ((p.Nq + 31) / 32) <= units) {
+  // Without a bias the items are of one size per head width, whatever the
+  // number of planes: an item keeps its fp16-weight pass, or an unshifted one,
+  // only where all of its rows allow it, so its size decides which rows hold
+  // fp16 weights and which hi + lo ones, and a row's company must not.  Four
+  // blocks per wave share a tile's staging and operand reads best at 64 dims
+  // (two at 128, by registers, and at 32, where a larger item is taken again
+  // as a whole for one row).  Smaller items are faster for some calls of few
+  // planes and slower for others: 64 planes of 1000 x 4096 x 64 119 us with four
+  // blocks and 132 with one where the fp16 pass holds, 251 and 218 where it does
+  // not; 32 of 3000 x 3000 126 and 113, 265 and 207.  (Smaller items whose
+  // groups agree through two further launches: 135 and 256, 117 and 231.)
+  if (p.bias == nullptr) {
+    switch (p.D) {
+      case 32: return launch_tile_k<T, OutT, 32, 64, 4, 2, false>(p, s);
+      case 64: return launch_tile_k<T, OutT, 64, 64, 4, 4, false>(p, s);
+      case 128: return launch_tile_k<T, OutT, 128, 32, 4, 2, false>(p, s);
+      default: return hipErrorInvalidValue;
+    }
+  }
+  // With a bias every path holds hi + lo weights, and the launch is chosen by
+  // time: a row's last bits in fp32 depend on how many planes share it.
+  // Few work items: the waves share out the keys instead of the queries, up to
+  // one 32-row item per CU (beyond, the streamed items gain more from the
+  // masked keys that they skip).  Measured, streamed and shared out, us: 176
+  // items of 700 masked keys 20 and 14, 352 of them 21 and 26.
+  if (planes * ((p.Nq + 31) / 32) <= units) {
     if (p.D == 32) return launch_span<T, OutT, 32>(p, units, s);
     if (p.D == 64) return launch_span<T, OutT, 64>(p, units, s);
     if (p.D == 128) return launch_span<T, OutT, 128>(p, units, s);
   }
-  // Query blocks per wave: four share a tile's staging and operand reads best
-  // (two for 128-dim heads, by registers, and 32-dim ones, where an item of 256
-  // rows is taken again as a whole when one row's fp16 weights may miss the
-  // bound), but the launch lasts as long as the fullest CU's items.  An item of
-  // four blocks per wave costs 1 / 0.57 of one of two.  Measured with 4 / 2 / 1,
-  // 64 dims, us: 256 planes of 4096 x 4096 1308 / 1547 / 2182, 64 of 2048 x 2048
-  // 193 / 214 / 265, 152 of 731 x 2882 262 / 279 / 288, 520 of 256 x 4096 284 /
-  // 267 / 319, 32 of 3000 x 3000 264 / 199 / 252, 64 of 1000 x 4096 206 / 164 /
-  // 153; 32 dims: 152 of 731 x 2882 193 / 148 / 177, 400 of 700 x 2000 319 / 335 / 381.
+  // Query blocks per wave: the launch lasts as long as the fullest CU's items,
+  // and an item of four blocks per wave costs 1 / 0.57 of one of two.
   switch (p.D) {
     case 32:
-      if (items(2) > units) return launch_tile_k<T, OutT, 32, 64, 4, 2>(p, s);
-      return launch_tile_k<T, OutT, 32, 64, 4, 1>(p, s);
+      if (items(2) > units) return launch_tile_k<T, OutT, 32, 64, 4, 2, true>(p, s);
+      return launch_tile_k<T, OutT, 32, 64, 4, 1, true>(p, s);
     case 64:
-      if (rounds(4) >= 2 && 100 * rounds(4) < 57 * rounds(2)) return launch_tile_k<T, OutT, 64, 64, 4, 4>(p, s);
-      if (2 * items(2) >= 5 * units) return launch_tile_k<T, OutT, 64, 64, 4, 2>(p, s);
-      return launch_tile_k<T, OutT, 64, 64, 4, 1>(p, s);
+      if (rounds(4) >= 2 && 100 * rounds(4) < 57 * rounds(2)) return launch_tile_k<T, OutT, 64, 64, 4, 4, true>(p, s);
+      if (2 * items(2) >= 5 * units) return launch_tile_k<T, OutT, 64, 64, 4, 2, true>(p, s);
+      return launch_tile_k<T, OutT, 64, 64, 4, 1, true>(p, s);
     case 128:
-      // Without a bias two always: where the fp16-weight pass is abandoned,
-      // items of one block are slower (3 planes of 930 x 3223 290 us, 211 with two).
-      if (p.bias == nullptr || items(2) > units) return launch_tile_k<T, OutT, 128, 32, 4, 2>(p, s);
-      return launch_tile_k<T, OutT, 128, 32, 4, 1>(p, s);
+      if (items(2) > units) return launch_tile_k<T, OutT, 128, 32, 4, 2, true>(p, s);
+      return launch_tile_k<T, OutT, 128, 32, 4, 1, true>(p, s);
     default: return hipErrorInvalidValue;
   }
 }
