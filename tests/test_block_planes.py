@@ -99,3 +99,21 @@ def test_planes_without_a_live_key_and_non_finite_masked_rows(n_k, dim):
     assert bool(got[1].isnan().all()) and not bool(got[0].isnan().any())
     assert bool(got[2, 0, :, 5].isnan().all()) and int(got[2, 0].isnan().sum()) == 50
     assert bool(got[2, 1].isnan().all())
+
+
+@pytest.mark.parametrize('n_q,n_k,dim,later', [(40, 257, 64, 200), (300, 300, 32, 299), (33, 150, 128, 40),  # staged whole
+                                               (40, 1200, 64, 512), (20, 1500, 32, 1030), (50, 400, 128, 256)])  # shared out
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16], ids=str)
+def test_what_the_split_drops_of_a_dominant_weight_drops_out(n_q, n_k, dim, later, dtype):
+    """Two live keys, the later one 120 times the weight the shift is taken
+    from: its hi + lo pair is 2^-17 off in bf16, and the sum it is divided by
+    holds the same pair.  Left: the fp32 roundings of the products, sums, the
+    reciprocal and its product (under 8 of 2^-24, the parts up to the values'
+    largest), and the logits' 2^-20 in the lighter key's hundredth."""
+    q, k, v, scale, _ = _inputs(2, 2, n_q, n_k, dim, dtype, 11)
+    b = torch.full((1, 1, 1, n_k), -math.inf)
+    b[..., 0], b[..., later] = 0.0, 4.8
+    got = _run(q, k, v, scale / 8, b)
+    want = torch.from_numpy(oracle.direct_fp64(q, k, v, scale / 8, b))
+    print(n_q, n_k, dim, dtype, float((got - want).abs().max()), flush=True)
+    torch.testing.assert_close(got, want, rtol=0, atol=8 * 2 ** -24 * float(v.float().abs().max()))

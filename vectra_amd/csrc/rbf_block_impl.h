@@ -12,8 +12,12 @@
 //   O^T = V^T . P^T   (16 value dims x 16 queries)
 //   x = coef (q.k - |q|^2 / 2) + c_j,  c_j = log2(e) (bias_j - gamma |k_j|^2)
 //
-// and weights go to the second product as hi + lo 16-bit pairs; their sum is
-// taken in fp32 on the vector unit.  Without a bias and with gamma >= 0 the
+// and weights go to the second product as hi + lo 16-bit pairs; a product of
+// the same pairs with ones divides it, so that what the split drops of a
+// dominant weight drops out, as in the tile kernel.  (The sum of the unsplit
+// weights on the vector unit took the same time, 27.2 us for the first shape
+// below, and left 1.2 to 1.7 times the error without a bias in fp16 and with
+// an additive one in bf16.)  Without a bias and with gamma >= 0 the
 // weights are used as they come (x <= 0); otherwise each query's weights are
 // shifted by its largest logit over the first 32 keys that count.  Where a
 // query's weight sum leaves the range in which the split is accurate (or a
@@ -37,7 +41,7 @@
 // (two passes, as masked planes took them) and here: 512 planes of 257 x 257 x
 // 64 76 and 25 us (HBM: 13), 1,600 of 100 x 100 x 64 81 and 23, 1,200 of
 // 130 x 130 x 128 110 and 55, 400 of 200 x 200 x 32 22 and 14.5.  Two query
-// blocks per wave (107 registers, four waves per SIMD, against 85) halve the
+// blocks per wave (107 registers, four waves per SIMD, against 88) halve the
 // operand reads and were 5-30% slower.
 
 #pragma once
@@ -181,6 +185,8 @@ rbf_block_kernel(Problem p, int32_t splits, int32_t blocks_per_split) {
   const bool plain = !has_bias && coef >= 0.f;
 
   // ---- The wave's query blocks.
+  const uint32_t one = Ops::kOnePair;
+  const Qk ones8 = __builtin_bit_cast(Qk, make_uint4(one, one, one, one));
   const char* qp = static_cast<const char*>(p.q) + (b * p.sq[0] + h * p.sq[1]) * 2;
   char* out_plane = static_cast<char*>(p.out) + (b * p.so[0] + h * p.so[1]) * static_cast<int64_t>(kOutSize);
   for (int32_t block = first_block + wave * kCB; block < end_block; block += kWaves * kCB) {
@@ -252,7 +258,7 @@ rbf_block_kernel(Problem p, int32_t splits, int32_t blocks_per_split) {
     };
 
     f32x4 acc[kCB][kDTiles];
-    float total[kCB];
+    f32x4 total[kCB];  // every row of the product with ones: the weight sum of the lane's query
 #pragma unroll
     for (int cb = 0; cb < kCB; ++cb) shift[cb] = 0.f;
     uint32_t max_pairs = plain ? 0u : (live & (0u - live));  // pairs the shift is taken over
@@ -260,7 +266,7 @@ rbf_block_kernel(Problem p, int32_t splits, int32_t blocks_per_split) {
       if (max_pairs != 0) largest(max_pairs);
 #pragma unroll
       for (int cb = 0; cb < kCB; ++cb) {
-        total[cb] = 0.f;
+        total[cb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int u = 0; u < kDTiles; ++u) acc[cb][u] = f32x4{0.f, 0.f, 0.f, 0.f};
       }
@@ -277,12 +283,13 @@ rbf_block_kernel(Problem p, int32_t splits, int32_t blocks_per_split) {
             float w[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) w[r] = __builtin_amdgcn_exp2f(x[cb][hb][r] - shift[cb]);
-            total[cb] += (w[0] + w[1]) + (w[2] + w[3]);
             Ops::split2(w[0], w[1], hi[2 * hb], lo[2 * hb]);
             Ops::split2(w[2], w[3], hi[2 * hb + 1], lo[2 * hb + 1]);
           }
           p_hi[cb] = __builtin_bit_cast(Qk, make_uint4(hi[0], hi[1], hi[2], hi[3]));
           p_lo[cb] = __builtin_bit_cast(Qk, make_uint4(lo[0], lo[1], lo[2], lo[3]));
+          total[cb] = Ops::qk(ones8, p_hi[cb], total[cb]);
+          total[cb] = Ops::qk(ones8, p_lo[cb], total[cb]);
         }
 #pragma unroll
         for (int u = 0; u < kDTiles; ++u) {
@@ -304,8 +311,7 @@ rbf_block_kernel(Problem p, int32_t splits, int32_t blocks_per_split) {
       bool off = false;
 #pragma unroll
       for (int cb = 0; cb < kCB; ++cb) {
-        total[cb] = allreduce_bit32(allreduce_bit16(total[cb], OpSum()), OpSum());
-        off = off || !(total[cb] >= kSumLo && (plain || total[cb] <= kSumHi));
+        off = off || !(total[cb][0] >= kSumLo && (plain || total[cb][0] <= kSumHi));
         if (!plain) {
 #pragma unroll
           for (int u = 0; u < kDTiles; ++u)
@@ -324,7 +330,7 @@ rbf_block_kernel(Problem p, int32_t splits, int32_t blocks_per_split) {
     for (int cb = 0; cb < kCB; ++cb) {
       const int32_t q_row = (block + cb) * 16 + col;
       if (block + cb >= end_block) continue;
-      const float inv = __builtin_amdgcn_rcpf(total[cb]);
+      const float inv = __builtin_amdgcn_rcpf(total[cb][0]);
       const uint32_t row_off = static_cast<uint32_t>(q_row) * o_row;
       if constexpr (kOutSize == 2) {
         if (out_vec) {

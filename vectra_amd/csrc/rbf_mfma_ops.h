@@ -59,6 +59,14 @@ struct MfmaOps<__bf16> {
     const float h0 = __uint_as_float(hi << 16), h1 = __uint_as_float(hi & 0xffff0000u);
     lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{w0 - h0, w1 - h1}, b2));
   }
+  // acc + the two elements of `pair` (one v_dot2; the ones come from a scalar
+  // register, as above).
+  static __device__ __forceinline__ float add2(uint32_t pair, float acc) {
+    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+    uint32_t ones;
+    asm("s_mov_b32 %0, 0x3f803f80" : "=s"(ones));
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(b2, pair), __builtin_bit_cast(b2, ones), acc, false);
+  }
 };
 
 template <>
@@ -86,6 +94,11 @@ struct MfmaOps<_Float16> {
   }
   static __device__ __forceinline__ void split2_sub(float w0, float w1, uint32_t& hi, uint32_t& lo) {
     split2(w0, w1, hi, lo);  // fp16: the v_dot2 form everywhere
+  }
+  static __device__ __forceinline__ float add2(uint32_t pair, float acc) {
+    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+    return __builtin_amdgcn_fdot2(__builtin_bit_cast(h2, pair),
+                                  h2{static_cast<_Float16>(1.f), static_cast<_Float16>(1.f)}, acc, false);
   }
 };
 

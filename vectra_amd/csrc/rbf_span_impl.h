@@ -22,9 +22,12 @@
 //
 // Bound: the vector unit (exp2, the split, the running shift) on the CUs that
 // have an item, with four waves per SIMD (two for 128-dim heads, by registers)
-// to cover a pair's chain.  Measured, bf16 with ragged masks, streamed tiles
-// and here: 8 planes of 700 x 700 x 64 20 and 14 us, of 1000 x 1000 x 64 26 and
-// 17, four of 640 x 640 x 128 29 and 12, 16 of 340 x 1300 x 32 23 and 11, four of
+// to cover a pair's chain.  The weight sum is that of the hi + lo pairs (see
+// rbf_block_impl.h), two per instruction after the products are issued: 1000 x
+// 1000 x 64 17.0 -> 18.0 us, as a product of ones 19.3 (16 registers spilled
+// for 12).  Measured, bf16 with ragged masks, streamed tiles
+// and here: 8 planes of 700 x 700 x 64 20 and 15 us, of 1000 x 1000 x 64 26 and
+// 18, four of 640 x 640 x 128 29 and 12, 16 of 340 x 1300 x 32 23 and 11, four of
 // 1000 x 2000 x 64 (fp16) 48 and 16.  Items of 16 queries where every CU holds
 // at most one: a plane of 1024 x 4096 x 64 25 us, 32 with items of 32.  Query
 // operands are read from LDS: in registers 25 more spilled at 64 dims.
@@ -225,7 +228,6 @@ __global__ __launch_bounds__(64 * span_waves<kD>()) void rbf_span_kernel(Problem
         float w[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) w[r] = __builtin_amdgcn_exp2f(x[hb][r] - off);
-        total[cb] += (w[0] + w[1]) + (w[2] + w[3]);
         Ops::split2(w[0], w[1], hi[2 * hb], lo[2 * hb]);
         Ops::split2(w[2], w[3], hi[2 * hb + 1], lo[2 * hb + 1]);
       }
@@ -246,6 +248,13 @@ __global__ __launch_bounds__(64 * span_waves<kD>()) void rbf_span_kernel(Problem
         acc[cb][u] = Ops::qk(a, p_hi[cb], acc[cb][u]);
         acc[cb][u] = Ops::qk(a, p_lo[cb], acc[cb][u]);
       }
+    }
+    // The sum of the same pairs, on the vector unit while the products run.
+#pragma unroll
+    for (int cb = 0; cb < kCB; ++cb) {
+      const uint4 hi = __builtin_bit_cast(uint4, p_hi[cb]), lo = __builtin_bit_cast(uint4, p_lo[cb]);
+      const float sum_lo = Ops::add2(lo.w, Ops::add2(lo.z, Ops::add2(lo.y, Ops::add2(lo.x, 0.f))));
+      total[cb] = Ops::add2(hi.w, Ops::add2(hi.z, Ops::add2(hi.y, Ops::add2(hi.x, total[cb] + sum_lo))));
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   }
