@@ -117,3 +117,18 @@ def test_what_the_split_drops_of_a_dominant_weight_drops_out(n_q, n_k, dim, late
     want = torch.from_numpy(oracle.direct_fp64(q, k, v, scale / 8, b))
     print(n_q, n_k, dim, dtype, float((got - want).abs().max()), flush=True)
     torch.testing.assert_close(got, want, rtol=0, atol=8 * 2 ** -24 * float(v.float().abs().max()))
+
+
+# A launch holds fewer than 2^32 threads: 2^22 workgroups of 16 waves, 2^24 of 4.
+@pytest.mark.parametrize('planes,n_k', [((1 << 22) + 5, 640), ((1 << 24) + 3, 81)])
+def test_more_planes_than_one_launch_holds(planes, n_k):
+    print(planes, n_k, flush=True)
+    q, k, v, scale = (t.contiguous().cuda() for t in _inputs(1, 1, 16, n_k, 32, torch.bfloat16, n_k)[:4])
+    bias = torch.zeros(planes, 1, 1, 1, dtype=torch.bfloat16, device='cuda')
+    bias[-1] = 1.0  # one value for all keys of a plane: no effect on its result
+    one = capi.forward(q, k, v, scale, bias[:1].expand(1, 1, 1, n_k))
+    out = torch.zeros(planes, 1, 16, 32, dtype=torch.bfloat16, device='cuda')
+    capi.forward(*(t.expand(planes, 1, -1, -1) for t in (q, k, v)), scale, bias.expand(planes, 1, 1, n_k), out=out)
+    torch.cuda.synchronize()
+    assert torch.equal(out[:-1], one.expand(planes - 1, 1, 16, 32))
+    torch.testing.assert_close(out[-1].float(), one[0].float(), rtol=2 ** -8, atol=1e-4)

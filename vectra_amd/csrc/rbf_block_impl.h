@@ -64,7 +64,7 @@ constexpr int64_t block_lds_bytes(int64_t n_k) {
 
 template <typename T, typename OutT, int kD, int kWaves>
 __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kD <= 64 ? 4 : 2))) void
-rbf_block_kernel(Problem p, int32_t splits, int32_t blocks_per_split) {
+rbf_block_kernel(Problem p, int32_t splits, int32_t blocks_per_split, int32_t first_plane) {
   using Ops = MfmaOps<T>;
   using Qk = typename Ops::Qk;
   constexpr int kCB = 1;  // query blocks a wave takes at a time (see above)
@@ -108,8 +108,9 @@ rbf_block_kernel(Problem p, int32_t splits, int32_t blocks_per_split) {
   const int32_t items = static_cast<int32_t>(gridDim.x);
   int32_t item = static_cast<int32_t>(blockIdx.x);
   if (items % 8 == 0) item = (item & 7) * (items / 8) + (item >> 3);
-  const int32_t bh = static_cast<int32_t>(fast_div(static_cast<uint32_t>(item), p.nq_mul, p.nq_shift));
-  const int32_t split = item - bh * splits;
+  const int32_t plane = static_cast<int32_t>(fast_div(static_cast<uint32_t>(item), p.nq_mul, p.nq_shift));
+  const int32_t split = item - plane * splits;
+  const int32_t bh = first_plane + plane;
   const int32_t b = static_cast<int32_t>(fast_div(static_cast<uint32_t>(bh), p.h_mul, p.h_shift));
   const int32_t h = bh - b * static_cast<int32_t>(p.H);
   const int32_t q_blocks = (n_q + 15) / 16;
@@ -379,11 +380,20 @@ template <typename T, typename OutT, int kD, int kWaves>
 hipError_t launch_block_k(Problem& p, int64_t splits, int64_t per_split, hipStream_t s) {
   Problem k = p;  // the kernel divides workgroups by the splits with the Nq slots
   make_fast_div(splits, &k.nq_mul, &k.nq_shift);
-  int32_t n = static_cast<int32_t>(splits), per = static_cast<int32_t>(per_split);
-  void* args[] = {&k, &n, &per};
-  return hipLaunchKernel(reinterpret_cast<const void*>(&rbf_block_kernel<T, OutT, kD, kWaves>),
-                         dim3(static_cast<unsigned>(p.B * p.H * splits)), dim3(64 * kWaves), args,
-                         static_cast<size_t>(block_lds_bytes<kD>(p.Nk)), s);
+  int32_t n = static_cast<int32_t>(splits), per = static_cast<int32_t>(per_split), first = 0;
+  void* args[] = {&k, &n, &per, &first};
+  // A grid holds fewer than 2^32 threads: very many planes take several
+  // launches (planes below 2^30: tile_supports).
+  const int64_t planes = p.B * p.H, most = 0xffffffffLL / (64 * kWaves) / splits;
+  for (int64_t plane = 0; plane < planes; plane += most) {
+    const int64_t here = planes - plane < most ? planes - plane : most;
+    first = static_cast<int32_t>(plane);
+    const hipError_t err = hipLaunchKernel(reinterpret_cast<const void*>(&rbf_block_kernel<T, OutT, kD, kWaves>),
+                                           dim3(static_cast<unsigned>(here * splits)), dim3(64 * kWaves), args,
+                                           static_cast<size_t>(block_lds_bytes<kD>(p.Nk)), s);
+    if (err != hipSuccess) return err;
+  }
+  return hipSuccess;
 }
 
 // Waves per workgroup by its LDS, so that the CU's workgroups together hold
@@ -406,7 +416,6 @@ hipError_t launch_block_d(Problem& p, hipStream_t s) {
   if (splits < 1) splits = 1;
   const int64_t per = (blocks + splits - 1) / splits;
   splits = (blocks + per - 1) / per;
-  if (planes * splits > 0x7fffffffLL) return hipErrorInvalidValue;
   if (waves == 16) return launch_block_k<T, OutT, kD, 16>(p, splits, per, s);
   if (waves == 8) return launch_block_k<T, OutT, kD, 8>(p, splits, per, s);
   return launch_block_k<T, OutT, kD, 4>(p, splits, per, s);
