@@ -41,6 +41,13 @@ def test_calls_that_keep_the_exact_forms():
     assert _bytes(num_queries=4) < 16 << 20 and _bytes(num_queries=1024, k=100) < 64 << 20
 
 
+@pytest.mark.parametrize('n_q', [2000, 65_536, 100_000, 1_000_000, 20_000_000])
+@pytest.mark.parametrize('k', [1, 10, 100, 512])
+def test_the_workspace_of_many_queries_is_bounded(n_q, k):
+    for rows in (8192, 100_000, 500_000):
+        assert 0 < _bytes(num_queries=n_q, k=k, num_rows=rows) <= 64 << 20, rows
+
+
 def _gpu(a):
     return torch.from_numpy(np.ascontiguousarray(a)).cuda()
 
@@ -78,6 +85,15 @@ def test_filtered_search_against_the_oracle(n_q, n, dim, k):
 @pytest.mark.parametrize('n_q,n,dim,k', [(64, 200_000, 128, 100), (9, 100_003, 64, 10), (1024, 12_500, 128, 100)])
 def test_filtered_search_at_large_sizes(n_q, n, dim, k):
     rng = np.random.default_rng(n)
+    _check(rng.standard_normal((n_q, dim)).astype(np.float32), rng.standard_normal((n, dim)).astype(np.float32), k,
+           against_oracle=False)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('n_q,n,dim,k', [(3001, 20_000, 32, 512), (7000, 6500, 64, 400)])
+def test_filtered_search_in_parts(n_q, n, dim, k):
+    """More queries than the workspace's bound holds at once: two and four parts."""
+    rng = np.random.default_rng(n_q)
     _check(rng.standard_normal((n_q, dim)).astype(np.float32), rng.standard_normal((n, dim)).astype(np.float32), k,
            against_oracle=False)
 

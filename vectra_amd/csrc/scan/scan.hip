@@ -1411,7 +1411,7 @@ int launch_top_k(int64_t queries, TopK& p, hipStream_t stream) {
 // and workspace, or bytes 0 where it does not apply.
 struct FilterPlan {
   TopKFilter f;
-  int64_t query_blocks = 0, bytes = 0;
+  int64_t queries = 0, query_blocks = 0, bytes = 0;  // of a part: the call runs in parts of `queries`
   int64_t minima = 0, limit = 0, counts = 0, lists = 0;  // byte offsets
 };
 
@@ -1426,6 +1426,13 @@ constexpr int64_t kFilterMinCands = 4096;
 constexpr int64_t kFilterQueriesAlone = 12;       // from here on whatever the candidates
 constexpr int64_t kFilterMinPairs = int64_t{1} << 17;  // below: this many (query, candidate) pairs
 
+// A call's workspace stays below this: more queries run in parts on it, one
+// after the other (the sample and the lists take up to 3 MB per 64 queries).
+constexpr int64_t kFilterMaxBytes = int64_t{64} << 20;
+
+// The plan of one part of `queries` queries, whatever its bytes.
+FilterPlan top_k_filter_part(int64_t queries, const TopK& p);
+
 FilterPlan top_k_filter_plan(int64_t queries, const TopK& p) {
   FilterPlan plan;
   if (queries < kFilterMinQueries || p.num_cand < kFilterMinCands || p.num_cand > 0x7fffffffLL ||
@@ -1434,7 +1441,18 @@ FilterPlan top_k_filter_plan(int64_t queries, const TopK& p) {
       reinterpret_cast<uintptr_t>(p.rows) % 16 != 0)
     return plan;
   const int64_t blocks = (queries + kFilterQueries - 1) / kFilterQueries;
-  if (blocks > kMaxBlocksY) return plan;
+  for (int64_t parts = 1; parts <= blocks; parts *= 2) {
+    const int64_t here = (blocks + parts - 1) / parts * kFilterQueries;
+    if (here > kMaxBlocksY * int64_t{kFilterQueries}) continue;
+    plan = top_k_filter_part(here < queries ? here : queries, p);
+    if (plan.bytes <= kFilterMaxBytes) break;
+  }
+  return plan;
+}
+
+FilterPlan top_k_filter_part(int64_t queries, const TopK& p) {
+  FilterPlan plan;
+  const int64_t blocks = (queries + kFilterQueries - 1) / kFilterQueries;
   TopKFilter& f = plan.f;
   f.t = p;
   f.num_queries = queries;
@@ -1475,6 +1493,7 @@ FilterPlan top_k_filter_plan(int64_t queries, const TopK& p) {
     plan.bytes += (bytes + 255) / 256 * 256;
     return at;
   };
+  plan.queries = queries;
   plan.query_blocks = blocks;
   take(kCounterBytes);  // the split form's counters stay as they are
   plan.minima = take(padded * waves * f.group_cols * static_cast<int64_t>(sizeof(float)));
@@ -1488,7 +1507,7 @@ template <bool kIds, int kChunks, int kTiles>
 int launch_top_k_filter(FilterPlan& plan, hipStream_t stream) {
   TopKFilter& f = plan.f;
   void* args[] = {&f};
-  const unsigned blocks = static_cast<unsigned>(plan.query_blocks);
+  const unsigned blocks = static_cast<unsigned>((f.num_queries + kFilterQueries - 1) / kFilterQueries);
   const int slabs = (f.t.dim + 32 * kChunks - 1) / (32 * kChunks);
   const size_t lds = static_cast<size_t>(slabs) * kChunks * kTiles * kWaveLanes * 16;
   auto go = [&](const void* kernel, dim3 grid, size_t bytes, unsigned threads = kFilterThreads) {
@@ -1519,17 +1538,27 @@ int launch_top_k_filter(FilterPlan& plan, hipStream_t stream) {
                                  : launch_top_k_filter<false, kChunks, kTiles>(plan, stream);
 }
 
-// Runs the filtered form on a workspace of at least plan.bytes.
-int run_top_k_filter(FilterPlan& plan, void* workspace, hipStream_t stream) {
+// Runs the filtered form on a workspace of at least plan.bytes, part by part.
+int run_top_k_filter(FilterPlan& plan, int64_t queries, void* workspace, hipStream_t stream) {
   char* base = static_cast<char*>(workspace);
   TopKFilter& f = plan.f;
   f.minima = reinterpret_cast<float*>(base + plan.minima);
   f.limit = reinterpret_cast<float*>(base + plan.limit);
   f.counts = reinterpret_cast<uint32_t*>(base + plan.counts);
   f.lists = reinterpret_cast<uint64_t*>(base + plan.lists);
-  const bool few = f.num_queries <= 16;
-  if (f.t.dim <= 64) return few ? launch_top_k_filter<2, 1>(plan, stream) : launch_top_k_filter<2, 4>(plan, stream);
-  return few ? launch_top_k_filter<4, 1>(plan, stream) : launch_top_k_filter<4, 4>(plan, stream);
+  const TopK all = f.t;
+  for (int64_t q = 0; q < queries; q += plan.queries) {
+    f.num_queries = queries - q < plan.queries ? queries - q : plan.queries;
+    f.t.queries = all.queries + q * all.query_stride;
+    f.t.distances = all.distances + q * all.out_stride;
+    f.t.nodes = all.nodes + q * all.out_stride;
+    const bool few = f.num_queries <= 16;
+    const int st = f.t.dim <= 64
+                       ? (few ? launch_top_k_filter<2, 1>(plan, stream) : launch_top_k_filter<2, 4>(plan, stream))
+                       : (few ? launch_top_k_filter<4, 1>(plan, stream) : launch_top_k_filter<4, 4>(plan, stream));
+    if (st != VECTRA_SCAN_OK) return st;
+  }
+  return VECTRA_SCAN_OK;
 }
 
 // Points the split form at a workspace: counters first, keys after.
@@ -1584,7 +1613,7 @@ extern "C" int vectra_scan_top_k_ws(const vectra_scan_top_k_args* a, void* works
     return VECTRA_SCAN_INVALID_ARGUMENT;
   FilterPlan plan = top_k_filter_plan(a->num_queries, p);
   if (plan.bytes > 0 && workspace != nullptr && workspace_bytes >= plan.bytes)
-    return run_top_k_filter(plan, workspace, stream);
+    return run_top_k_filter(plan, a->num_queries, workspace, stream);
   const int64_t splits = top_k_splits(a->num_queries, p);
   if (splits > 1 && workspace != nullptr && workspace_bytes >= top_k_workspace(a->num_queries, splits, p.k))
     use_workspace(p, splits, workspace);
