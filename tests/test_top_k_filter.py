@@ -160,3 +160,50 @@ def test_a_smaller_workspace_takes_the_exact_forms():
         got = scan.nearest(q, rows, 20, workspace=torch.zeros(size, dtype=torch.uint8, device='cuda'))
         torch.cuda.synchronize()
         assert all(torch.equal(a.view(torch.int32), b.view(torch.int32)) for a, b in zip(got, want)), size
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('k', [10, 200])
+def test_lists_that_keep_their_smallest_keys(k):
+    """The nearest candidates in one or two workgroups' shares: their lists run
+    over, and what they left out is among the k nearest; equal keys of one node
+    beyond a list's slots; equal distances of many nodes."""
+    rng = np.random.default_rng(k)
+    n, dim = 9000, 64
+    q = rng.standard_normal((16, dim)).astype(np.float32)
+    rows = rng.standard_normal((n, dim)).astype(np.float32)
+    ahead = rows[np.argsort(((rows - q[3]) ** 2).sum(1))]
+    for name, data, ids in (('sorted', ahead, None), ('reversed', ahead[::-1].copy(), None),
+                            ('one_node', rows, np.full(6000, 7)), ('few_nodes', rows, rng.integers(0, 5, 6000)),
+                            ('runs', rows[np.arange(n) // 300], None), ('runs_of_ids', rows, np.arange(9000) // 40)):
+        print(name, k, flush=True)
+        _check(q, data, k, ids)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('kind', ['equal', 'two_values'])
+def test_ties_cost_no_multiple_of_the_exact_search(kind):
+    """Every list of every query runs over: without its smallest keys each
+    query's candidates were computed again by one workgroup, five times the
+    exact form's time in all."""
+    gen = torch.Generator(device='cuda').manual_seed(1)
+    rows = torch.randn(60_000, 128, generator=gen, device='cuda')
+    q = torch.randn(64, 128, generator=gen, device='cuda')
+    rows[:] = rows[:1] if kind == 'equal' else rows[:2].repeat(30_000, 1)
+    workspace = torch.zeros(scan.workspace_bytes(q, rows, 100), dtype=torch.uint8, device='cuda')
+
+    def time(**kw):
+        best = float('inf')
+        for _ in range(4):
+            begin, end = torch.cuda.Event(True), torch.cuda.Event(True)
+            begin.record()
+            for _ in range(5):
+                scan.nearest(q, rows, 100, **kw)
+            end.record()
+            torch.cuda.synchronize()
+            best = min(best, begin.elapsed_time(end))
+        return best
+
+    filtered, exact = time(workspace=workspace), time(form='single')
+    print(f'{kind}: filtered {filtered:.3f} ms, exact {exact:.3f} ms', flush=True)
+    assert filtered < 2.5 * exact

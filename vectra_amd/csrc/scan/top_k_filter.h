@@ -23,8 +23,9 @@
 //     not above the limit are computed exactly, and the ones at or below
 //     the limit go into the workgroup's short list of the query;
 //  4. top_k_merge_kernel: per query, the k smallest keys of the lists.  A list
-//     that ran over (ties, clustered data) is replaced by an exact scan of
-//     its workgroup's candidates.
+//     that runs over (ties, loose bounds) keeps its smallest keys, so what it
+//     left out is no nearer than the last of them: its workgroup's candidates
+//     are scanned again only where that key is below the k-th found.
 //
 // The results are those of scan_top_k_kernel, bit for bit: every returned
 // distance is the reference's arithmetic, and a candidate is dropped only
@@ -60,7 +61,7 @@ struct TopKFilter {
   float* minima;     // [query blocks][groups][64]
   float* limit;      // [query blocks][64]
   uint32_t* counts;  // [query blocks][workgroups][64]; above kFilterCap: ran over
-  uint64_t* lists;   // [query blocks][workgroups][64][kFilterCap]
+  uint64_t* lists;   // [query blocks][workgroups][64][kFilterCap]; of one that ran over, its smallest keys
   int64_t num_queries;
   int32_t tiles;         // 16-candidate tiles of the call
   int32_t workgroups;    // of the filter launch, per query block
@@ -89,6 +90,53 @@ __device__ __forceinline__ float dpp_min(float x, C) {
 template <typename C>
 __device__ __forceinline__ float dpp_add(float x, C) {
   return x + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), C::value, 0xf, 0xf, false));
+}
+
+// A key in LDS that other waves change meanwhile.
+__device__ __forceinline__ uint64_t shared_key(const uint64_t* key) {
+  return __hip_atomic_load(key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// Puts `key` into a full list of kFilterCap keys in LDS in place of its largest,
+// for each 16-lane group with `left` (the lanes of a group hold a slot each);
+// other waves insert at the same time.  A slot that still reads as empty
+// (kNoKey) has been given to a wave that is about to write it: look again.
+// Written slots only ever fall, so a key found no smaller than every slot, or
+// replaced as the largest, is no smaller than any key the list ends with;
+// `worst` is such a bound, above which no look at the slots is needed.
+//
+// The whole wave runs this and each of its rounds: conditions are computed
+// without branches (&, unconditional loads), as lanes that the compiler takes
+// around a load could otherwise reach a ballot apart from the rest.
+__device__ __forceinline__ void list_replace(uint64_t* list, uint64_t* worst, uint64_t key, bool left, int lane,
+                                             int wave_lane) {
+  static_assert(kFilterCap == kLanes, "a lane per slot");
+  typedef unsigned long long Word;
+  const int group_bit = wave_lane & ~(kLanes - 1);
+  // (`worst` is told of lists that have run over only: what it keeps out is not counted.)
+  const bool tells = left & (lane == 0);
+  do {
+    const uint64_t slot = shared_key(list + lane);
+    uint64_t largest = slot;
+    auto fold = [&](auto s_tag) {
+      const uint64_t other = lane_xor<decltype(s_tag)::value>(largest, wave_lane);
+      largest = other > largest ? other : largest;
+    };
+    fold(std::integral_constant<int, 1>{});
+    fold(std::integral_constant<int, 2>{});
+    fold(std::integral_constant<int, 4>{});
+    fold(std::integral_constant<int, 8>{});
+    const bool whole = largest != kNoKey;
+    left = left & (key < largest);
+    const bool placing = left & whole;
+    // The first lane whose slot is the largest.
+    const uint64_t holders = (__ballot(placing & (slot == largest)) >> group_bit) & 0xffffu;
+    const bool mine = placing & (((holders >> lane) & 1) != 0) & ((holders & ((uint64_t{1} << lane) - 1)) == 0);
+    bool put = false;
+    if (mine) put = atomicCAS(reinterpret_cast<Word*>(list) + lane, static_cast<Word>(largest), static_cast<Word>(key)) == largest;
+    if (tells & whole) atomicMin(reinterpret_cast<Word*>(worst), static_cast<Word>(largest));
+    left = left & (((__ballot(put) >> group_bit) & 0xffffu) == 0);
+  } while (__ballot(left) != 0);
 }
 
 // The exact distance of kN (query, row) pairs of this 16-lane group, in the
@@ -147,6 +195,7 @@ __global__ __launch_bounds__(kFilterThreads, kSample ? 4 : 3) void top_k_bound_k
   __shared__ __align__(16) float qa[kFilterQueries], qc[kFilterQueries];
   __shared__ float qlimit[kFilterQueries];
   __shared__ uint32_t fill[kFilterQueries];
+  __shared__ uint64_t worst[kSample ? 1 : kFilterQueries];
   __shared__ uint64_t list[kSample ? 1 : kFilterQueries][kSample ? 1 : kFilterCap];
   __shared__ uint32_t queue[kSample ? 1 : kFilterWaves][kSample ? 1 : kFilterQueue];
 
@@ -213,7 +262,11 @@ __global__ __launch_bounds__(kFilterThreads, kSample ? 4 : 3) void top_k_bound_k
       qa[tid] = tid < nq ? 0.5f * (n * (1.f - c2) - limit - 1e-30f) : INFINITY;
       qc[tid] = 0.5f * c1 * length;
       fill[tid] = 0u;
+      worst[tid] = kNoKey;
     }
+  }
+  if constexpr (!kSample) {
+    for (int s = tid; s < kFilterQueries * kFilterCap; s += kFilterThreads) list[s / kFilterCap][s % kFilterCap] = kNoKey;
   }
   __syncthreads();
 
@@ -262,6 +315,11 @@ __global__ __launch_bounds__(kFilterThreads, kSample ? 4 : 3) void top_k_bound_k
     for (int r = 0; r < 4; ++r) best[t][r] = INFINITY;
   int queued = 0;  // survivors in the wave's queue (wave-uniform)
 
+  // Fills slot `pos` of query q's list.
+  auto put_key = [&](int q, uint32_t pos, uint64_t key) {
+    __hip_atomic_store(&list[kSample ? 0 : q][kSample ? 0 : pos], key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  };
+
   // Computes the queued pairs exactly and lists those at or below the limit.
   auto drain = [&]() {
     constexpr int kPairs = 4;
@@ -284,12 +342,32 @@ __global__ __launch_bounds__(kFilterThreads, kSample ? 4 : 3) void top_k_bound_k
       }
       float sum[kPairs];
       exact_distances<kPairs>(query, row, dim, col, sum);
+      // Into the lists (fill counts the keys offered): a slot of the key's own,
+      // or, where the list is full, the largest key's.
+      bool want[kPairs];
+      uint32_t pos[kPairs];
 #pragma unroll
       for (int n = 0; n < kPairs; ++n) {
-        if (col == 0 && e0 + n * 4 + grp < queued && q[n] < nq && !(sum[n] > qlimit[q[n]])) {
-          const uint32_t pos = atomicAdd(&fill[q[n]], 1u);
-          if (pos < kFilterCap) list[kSample ? 0 : q[n]][kSample ? 0 : pos] = nearest_key(sum[n], node[n]);
-        }
+        want[n] = (col == 0) & (e0 + n * 4 + grp < queued) & (q[n] < nq) & !(sum[n] > qlimit[q[n]]);
+        pos[n] = kFilterCap;
+        if (want[n]) pos[n] = atomicAdd(&fill[q[n]], 1u);
+      }
+      bool full = false;
+#pragma unroll
+      for (int n = 0; n < kPairs; ++n) {
+        if (pos[n] < static_cast<uint32_t>(kFilterCap)) put_key(q[n], pos[n], nearest_key(sum[n], node[n]));
+        want[n] = want[n] & (pos[n] >= static_cast<uint32_t>(kFilterCap));
+        full = full | want[n];
+      }
+      if (__ballot(full) == 0) continue;
+#pragma unroll
+      for (int n = 0; n < kPairs; ++n) {
+        const uint64_t key = nearest_key(sum[n], node[n]);
+        uint64_t* bound = &worst[kSample ? 0 : q[n]];
+        const bool left = want[n] & (key < shared_key(bound));
+        if (__ballot(left) == 0) continue;
+        list_replace(list[kSample ? 0 : q[n]], bound, __shfl(key, 0, kLanes), __shfl(static_cast<int>(left), 0, kLanes) != 0,
+                     col, lane);
       }
     }
     queued = 0;
@@ -527,8 +605,9 @@ __device__ __forceinline__ void sort_keys_by_wave(uint64_t* keys, int n, int tid
 template <bool kIds, int kMergeThreads>
 __global__ __launch_bounds__(kMergeThreads) void top_k_merge_kernel(TopKFilter p) {
   __shared__ uint64_t keys[kTopKKeys];  // the k best so far (none at first), then new ones
-  __shared__ uint32_t fill, over_count;
-  __shared__ uint32_t over[kFilterMaxWorkgroups];  // workgroups whose list ran over
+  __shared__ uint32_t fill, over_count, equal;
+  __shared__ uint32_t over[kFilterMaxWorkgroups];  // workgroups whose list ran over ...
+  __shared__ uint64_t over_last[kFilterMaxWorkgroups];  // ... and their lists' largest keys
   const int tid = static_cast<int>(threadIdx.x);
   const int64_t query = blockIdx.x;
   const int64_t block = query / kFilterQueries;
@@ -543,8 +622,15 @@ __global__ __launch_bounds__(kMergeThreads) void top_k_merge_kernel(TopKFilter p
     const int64_t at = (block * p.workgroups + w) * kFilterQueries + q;
     uint32_t n = w < p.workgroups ? p.counts[at] : 0u;
     if (n > static_cast<uint32_t>(kFilterCap)) {
-      over[atomicAdd(&over_count, 1u)] = static_cast<uint32_t>(w);
-      n = 0;
+      n = kFilterCap;
+      uint64_t last = 0;
+      for (uint32_t s = 0; s < n; ++s) {
+        const uint64_t x = p.lists[at * kFilterCap + s];
+        last = x > last ? x : last;
+      }
+      const uint32_t o = atomicAdd(&over_count, 1u);
+      over[o] = static_cast<uint32_t>(w);
+      over_last[o] = last;
     }
     bool pending = n > 0;
     while (true) {
@@ -576,23 +662,33 @@ __global__ __launch_bounds__(kMergeThreads) void top_k_merge_kernel(TopKFilter p
     __syncthreads();
   }
 
-  // The candidates of workgroups whose list ran over, 64 at a time: the
-  // first 16 16-lane groups compute four each.
+  // Workgroups whose list ran over with its largest key below the k-th found:
+  // their candidates once more, the keys above that largest (and, of those
+  // equal to it, the ones the list left out), kMergeThreads / 4 at a time: a
+  // 16-lane group computes four.
   const int n_over = static_cast<int>(over_count);
   const int lane = tid & (kLanes - 1);
   const int group = tid / kLanes;
+  constexpr int kStripes = kMergeThreads / kFilterThreads;  // of 64 candidates
   const float* qrow = p.t.queries + query * p.t.query_stride;
   for (int o = 0; o < n_over; ++o) {
-    for (int64_t first = static_cast<int64_t>(over[o]) * 64; first < p.t.num_cand;
-         first += static_cast<int64_t>(p.workgroups) * 64) {
+    const uint64_t last = over_last[o];
+    if (last >= keys[k - 1]) continue;  // uniform: the keys were sorted behind a barrier
+    const int64_t w = over[o];
+    const uint64_t* held_keys = p.lists + ((block * p.workgroups + w) * kFilterQueries + q) * kFilterCap;
+    uint32_t last_held = 0;
+    for (int e = 0; e < kFilterCap; ++e) last_held += held_keys[e] == last;
+    if (tid == 0) equal = 0u;
+    __syncthreads();
+    for (int64_t first = w * 64; first < p.t.num_cand; first += static_cast<int64_t>(p.workgroups) * 64 * kStripes) {
       const float* query4[4];
       const float* row4[4];
       uint32_t node[4];
       bool ok[4];
 #pragma unroll
       for (int n = 0; n < 4; ++n) {
-        const int64_t cand = first + (group & 15) * 4 + n;
-        ok[n] = group < 16 && cand < p.t.num_cand;
+        const int64_t cand = first + static_cast<int64_t>(group / 16) * p.workgroups * 64 + (group & 15) * 4 + n;
+        ok[n] = cand < p.t.num_cand;
         node[n] = ok[n] ? static_cast<uint32_t>(cand) : 0u;
         if constexpr (kIds) {
           node[n] = ok[n] ? p.t.ids[cand] : 0u;
@@ -604,27 +700,31 @@ __global__ __launch_bounds__(kMergeThreads) void top_k_merge_kernel(TopKFilter p
       }
       float sum[4];
       exact_distances<4>(query4, row4, p.t.dim, lane, sum);
+      const uint64_t kth = keys[k - 1];
 #pragma unroll
       for (int n = 0; n < 4; ++n) {
         if (ok[n] && lane == 0) {
           const uint64_t key = nearest_key(sum[n], node[n]);
-          if (key < keys[k - 1]) keys[k + atomicAdd(&fill, 1u)] = key;
+          if (key < kth && (key > last || (key == last && atomicAdd(&equal, 1u) >= last_held)))
+            keys[k + atomicAdd(&fill, 1u)] = key;
         }
       }
       __syncthreads();
       const int n = static_cast<int>(fill);
       __syncthreads();
-      if (n + 64 > kTopKKeys - k || (n > 0 && keys[k - 1] == kNoKey)) {
+      if (n + 64 * kStripes > kTopKKeys - k || (n > 0 && kth == kNoKey)) {
         sort_keys_by_wave<kMergeThreads>(keys, k + n, tid);
         if (tid == 0) fill = 0u;
         __syncthreads();
       }
     }
-  }
-  if (n_over > 0) {
     const int n = static_cast<int>(fill);
     __syncthreads();
-    if (n > 0) sort_keys_by_wave<kMergeThreads>(keys, k + n, tid);
+    if (n > 0) {
+      sort_keys_by_wave<kMergeThreads>(keys, k + n, tid);
+      if (tid == 0) fill = 0u;
+      __syncthreads();
+    }
   }
   for (int r = tid; r < k; r += kMergeThreads) {
     const uint64_t key = keys[r];
