@@ -69,3 +69,36 @@ def test_rows_do_not_depend_on_the_planes_beside_them(n_q, n_k, dim, out_dtype):
         print(planes, n_q, n_k, dim, flush=True)
         many = capi.forward(*(t.expand(planes, -1, -1, -1) for t in (q, k, v)), scale, out_dtype=out_dtype, variant='tile')
         assert torch.equal(many, alone.expand_as(many)), planes
+
+
+def test_keys_padded_on_the_left_take_one_pass():
+    """Where the first tiles are masked whole, the shift comes from the first
+    that is not: a shift of 0 leaves these weight sums under fp16's range, and
+    the planes took three passes (padded on the right: one)."""
+    planes, n_q, n_k, dim = 256, 512, 1024, 64
+    gen = torch.Generator(device='cuda').manual_seed(0)
+    q, k, v = (torch.randn(planes, 1, n, dim, generator=gen, device='cuda').half() for n in (n_q, n_k, n_k))
+    scale = torch.full((1, 1, 1, 1), 0.15, device='cuda')
+    bias = torch.zeros(planes, 1, 1, n_k, device='cuda')
+    bias[..., :200] = -math.inf
+
+    def run(keys, values, mask):
+        best = math.inf
+        for _ in range(4):
+            begin, end = torch.cuda.Event(True), torch.cuda.Event(True)
+            begin.record()
+            for _ in range(5):
+                out = capi.forward(q, keys, values, scale, mask, out_dtype=torch.float32, variant='tile')
+            end.record()
+            torch.cuda.synchronize()
+            best = min(best, begin.elapsed_time(end))
+        return out, best
+
+    left, left_ms = run(k, v, bias)
+    right, right_ms = run(k.flip(2), v.flip(2), bias.flip(3))
+    print(f'padded on the left {left_ms:.3f} ms, on the right {right_ms:.3f} ms', flush=True)
+    # The shifts differ, and with them what fp16's last step of 2^-24 cuts from
+    # 824 weights of a sum of at least 2^-3: up to 2^-22 of the sum each, as a
+    # walk (four deviations of sqrt(824) 2^-22 / sqrt(3)) against |v| < 6.
+    torch.testing.assert_close(left, right, rtol=0, atol=1e-4)
+    assert left_ms < 1.6 * right_ms

@@ -526,8 +526,9 @@ rbf_tile_kernel(Problem p, int32_t q_blocks) {
   };
   Stage st;
   int32_t parity = 0;
-  // A shifted pass with `guess` takes the first tile's largest logits as its
-  // shift.
+  // A shifted pass with `guess` takes as its shift the largest logits of the
+  // first tile with a key that counts, and starts there (shifted by tile 0,
+  // left-padded fp16 planes of far logits took three passes).
   auto run_pass = [&](const Coords& c, float coef, bool active, bool guess, auto kind_c) __attribute__((always_inline)) {
     constexpr bool kFast = decltype(kind_c)::value == kPassFast;
     if constexpr (decltype(kind_c)::value != kPassMax) {
@@ -547,14 +548,30 @@ rbf_tile_kernel(Problem p, int32_t q_blocks) {
     issue(st, c, 0);
     publish(st, 0, 0, coef, kind_c);
     __syncthreads();
-    if (tiles > 1) issue(st, c, 1);
+    int32_t t0 = 0;  // the pass's first tile
+    if constexpr (kBias && decltype(kind_c)::value == kPassShifted) {
+      // Tiles without a key that counts, up to the first that has one.
+      auto dead = [&]() __attribute__((always_inline)) {
+        bool live = false;
+#pragma unroll
+        for (int kp = 0; kp < G::kPairs; ++kp) live = live || pair_live(t0 & 1, t0, kp);
+        return !live;
+      };
+      while (guess && t0 + 1 < tiles && dead()) {
+        ++t0;
+        issue(st, c, t0);
+        publish(st, t0, t0 & 1, coef, kind_c);
+        __syncthreads();
+      }
+    }
+    if (t0 + 1 < tiles) issue(st, c, t0 + 1);
     const int32_t probe = tiles / 8;  // tiles reduced when the fast pass checks its course
-    for (int32_t t = 0; t < tiles; ++t) {
+    for (int32_t t = t0; t < tiles; ++t) {
       if constexpr (kBias) {
         if (active) {
           if constexpr (decltype(kind_c)::value == kPassShifted) {
-            if (guess && t == 0) {
-              compute(0, 0, coef, PassKind<kPassMax>{});
+            if (guess && t == t0) {
+              compute(t & 1, t, coef, PassKind<kPassMax>{});
               settle_max();
             }
           }
@@ -621,7 +638,7 @@ rbf_tile_kernel(Problem p, int32_t q_blocks) {
       return exact_flag[parity] != 0;
     };
     bool exact = true;   // passes are left to do
-    bool guess = false;  // ... the next one shifted by the first tile's largest logits
+    bool guess = false;  // ... the next one shifted by one tile's largest logits
     if constexpr (kBias) {
       guess = true;
     } else if (coef >= 0.f) {  // the unshifted passes need x <= 0
@@ -654,7 +671,7 @@ rbf_tile_kernel(Problem p, int32_t q_blocks) {
         exact = redo_item(low);
       }
     }
-    // With a bias, one pass shifted by the first tile's largest logits; where
+    // With a bias, one pass shifted by one tile's largest logits; where
     // that leaves the range, and for gamma < 0, the exact passes: each query's
     // largest logit, then the pass shifted by it.
     while (exact) {
