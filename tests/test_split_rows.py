@@ -77,3 +77,21 @@ def test_split_rows_without_a_live_key_are_nan():
     out = torch.ops.vectra.rbf_attention(q, k, v, torch.tensor(0.01, device='cuda'), bias)
     torch.cuda.synchronize()
     assert bool(out[1].isnan().all()) and not bool(out[0].isnan().any())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('rows', [4, 4096])  # 16 waves and one wave per row
+def test_split_rows_of_equal_keys_are_exact(rows):
+    """Every weight is exactly 1, so sums and counts are whole numbers and each
+    result is their exact quotient (a product with the rounded reciprocal of
+    49 or 93 keys is not)."""
+    off = []
+    for n_k in (65, 93, 98, 123, 161, 186, 196, 333, 509):
+        q = torch.ones(rows, 1, 1, 64, device='cuda')
+        k = torch.ones(rows, 1, n_k, 64, device='cuda')
+        v = torch.full((rows, 1, n_k, 64), 3.0, device='cuda')
+        got = torch.ops.vectra.rbf_attention(q, k, v, torch.tensor(0.5, device='cuda'), None)
+        torch.cuda.synchronize()
+        if not bool((got == 3.0).all()):
+            off.append(n_k)
+    assert not off

@@ -487,10 +487,10 @@ __global__ __launch_bounds__(kSplitMaxWaves * kWave) void rbf_split_kernel(Probl
   // Row groups below lane bit 16 hold copies; one of them writes.
   const bool writer = kChunks >= 16 || (lane & (16 - kChunks)) == 0;
   if (n_waves == 1) {
-    // A row whose keys are all masked has sum 0: 0 * inf = NaN, as eager.
-    const float inv = __builtin_amdgcn_rcpf(wave_sum);
+    // A quotient, as the generic kernel has it (the reciprocal's rounding adds
+    // one more).  A row whose keys are all masked is 0 / 0 = NaN, as eager.
 #pragma unroll
-    for (int i = 0; i < kOut; ++i) res[i] *= inv;
+    for (int i = 0; i < kOut; ++i) res[i] /= wave_sum;
     if (writer) store_small<OutT, kOut>(out + chunk * kVec + first_e, res);
     return;
   }
@@ -515,7 +515,7 @@ __global__ __launch_bounds__(kSplitMaxWaves * kWave) void rbf_split_kernel(Probl
       sum = fmaf(f, part_sum[w0 + w], sum);
       value = fmaf(f, part_acc[w0 + w][d], value);
     }
-    out[d] = from_float<OutT>(value * __builtin_amdgcn_rcpf(sum));
+    out[d] = from_float<OutT>(value / sum);
   }
 }
 
