@@ -394,11 +394,15 @@ __global__ __launch_bounds__(kSplitMaxWaves * kWave) void rbf_split_kernel(Probl
       load16(reinterpret_cast<const char*>(p.q) + (c.b * p.sq[0] + c.h * p.sq[1] + c.i * p.sq[2]) * sizeof(T) +
              chunk_bytes);
   const RawScalar scale_raw = load_raw_scalar(p.scale, c.b * p.ssb + c.h * p.ssh, p.scale_dtype);
-  // The row's tile order is rotated by a hash of the row: where planes are a
+  // The row's tile order is rotated by a hash of its plane: where planes are a
   // power of two apart, waves that walk them in step from the first tile
   // would all be on the same few HBM channels (8192 rows of 256 keys: 41.9 us
-  // rotated, 51.2 in order).
-  const int32_t rotation = static_cast<int32_t>(__umulhi(static_cast<uint32_t>(row) * 0x9e3779b1u, tiles));
+  // rotated, 51.2 in order).  The rows of a plane walk it in one order and
+  // meet its tiles in the caches (rotated row by row, 2000 planes of 3 rows x
+  // 500 keys took 51.2 us in fp32 at 16 dims, now 38.3; of 15 rows x 300 at 64
+  // dims 529 and 323).
+  const uint32_t plane = static_cast<uint32_t>(c.b * p.H + c.h);
+  const int32_t rotation = static_cast<int32_t>(__umulhi(plane * 0x9e3779b1u, tiles));
   auto rotated = [&](int32_t t) { return t + rotation < tiles ? t + rotation : t + rotation - tiles; };
   int32_t step = wave, tile = rotated(step);
   if (step < tiles) issue(a, tile);
