@@ -50,3 +50,23 @@ def test_non_finite_rows_of_masked_fp32_keys_reach_the_output():
     out = capi.forward(q.cuda(), k.cuda(), v.cuda(), torch.tensor(0.01).cuda(), bias2.cuda(), variant='mfma').cpu()
     assert bool(out[0, 0, :, 7].isnan().all()) and int(out[0, 0].isnan().sum()) == 90
     assert bool(out[0, 1].isnan().all()) and bool(out[0, 2].isnan().all())
+
+
+# Both sides of the rule on waves per workgroup for 65-80 rows and beyond, by
+# planes and key count, at 256 compute units.
+@pytest.mark.parametrize('planes,n_q,n_k,dim', [(150, 65, 90, 64), (160, 80, 90, 64), (330, 80, 130, 64), (520, 65, 130, 64),
+                                                (520, 80, 170, 64), (160, 70, 70, 128), (520, 66, 40, 128), (150, 81, 100, 64),
+                                                (160, 128, 100, 64), (330, 113, 70, 128)])
+def test_many_masked_fp32_planes(planes, n_q, n_k, dim):
+    print(planes, n_q, n_k, dim, flush=True)
+    g = torch.Generator(device='cuda').manual_seed(planes + n_q)
+    q, k, v = (torch.randn(planes, 1, n, dim, generator=g, device='cuda') for n in (n_q, n_k, n_k))
+    scale = torch.full((1, 1, 1, 1), 0.9 / dim, device='cuda')
+    counts = torch.randint(1, n_k + 1, (planes, 1, 1, 1), generator=g, device='cuda')
+    bias = torch.zeros(planes, 1, 1, n_k, device='cuda')
+    bias.masked_fill_(torch.arange(n_k, device='cuda') >= counts, -math.inf)
+    got = capi.forward(q, k, v, scale, bias, variant='mfma')
+    qd, kd, vd = (t[:, 0].double() for t in (q, k, v))
+    d2 = (qd * qd).sum(-1)[..., None] + (kd * kd).sum(-1)[:, None] - 2 * (qd @ kd.transpose(1, 2).contiguous())
+    want = torch.softmax(bias[:, 0].double() - scale.double().item() * d2, -1) @ vd
+    torch.testing.assert_close(got[:, 0].double(), want, rtol=1e-5, atol=1e-5)

@@ -564,19 +564,31 @@ hipError_t launch_mfma_w(Problem& p, hipStream_t s) {
 // Waves per workgroup: one per 16-row query tile of a plane, at least 4 (the
 // loaders' register staging of a tile is split over the workgroup) and at
 // most 8; 5 covers the 65-token comparable sets.  fp32 with a bias takes 4
-// where 8 would leave CUs idle, and from 1.25 items of 8 waves per CU on
-// (finer ones balance ragged planes): 8 planes of 900 x 900 x 64 74 us with 8
-// waves and 58 with 4, 320 of 120 x 120 x 64 29 and 26, 180 of 431 x 431 x 32
-// 66 and 61; about one item of 8 waves per CU stays with 8 (64 planes of
-// 500 x 500 x 64 48 and 52).
+// where 8 would leave two fifths of the CUs idle, and from 1.25 items of 8
+// waves per CU on (finer ones balance ragged planes); 8 and 4 waves, us: 8
+// planes of 900 x 900 x 64 74 and 58, 140 of 120 x 120 x 64 15.3 and 13.4, 180
+// of 128 x 128 x 128 31 and 36, 64 of 500 x 500 x 64 48 and 52, 320 of
+// 120 x 120 x 64 29 and 26, 180 of 431 x 431 x 32 66 and 61.  65-80 rows are
+// two items of 4 waves, one of them with a single row tile, instead of one of 5
+// only where CUs would idle or few planes or long key axes leave more to
+// balance than the second staging costs; 5 and 4 waves, us: 128 planes of
+// 70 x 70 x 64 12.9 and 10.8, 190 of 70 x 70 x 128 22 and 26, 320 of
+// 65 x 65 x 64 22.8 and 21.2, 600 of 80 x 600 x 64 160 and 136; 512 of
+// 80 x 80 x 128 44 and 49, 2000 of 65 x 65 x 64 81 and 84.
 template <typename T, typename OutT, int kD, int kKeys>
 hipError_t launch_mfma_k(Problem& p, hipStream_t s) {
   const int64_t tiles = (p.Nq + 15) / 16;
   const int64_t units = p.compute_units > 0 ? p.compute_units : 1;
   const int64_t items = p.B * p.H * ((tiles + 7) / 8);
-  const bool small = sizeof(T) == 4 && p.bias != nullptr && (4 * items < 3 * units || 4 * items >= 5 * units);
-  if (tiles <= 4 || small) return launch_mfma_w<T, OutT, kD, kKeys, 4>(p, s);
-  if (tiles <= 5) return launch_mfma_w<T, OutT, kD, kKeys, 5>(p, s);
+  const bool fine = sizeof(T) == 4 && p.bias != nullptr;
+  const bool idle = 5 * items < 3 * units, ragged = 4 * items >= 5 * units;
+  if (tiles <= 4) return launch_mfma_w<T, OutT, kD, kKeys, 4>(p, s);
+  if (tiles == 5) {
+    const bool two = fine && (idle || (ragged && (items < 2 * units || p.Nk > 160)));
+    if (!two) return launch_mfma_w<T, OutT, kD, kKeys, 5>(p, s);
+    return launch_mfma_w<T, OutT, kD, kKeys, 4>(p, s);
+  }
+  if (fine && (idle || ragged)) return launch_mfma_w<T, OutT, kD, kKeys, 4>(p, s);
   return launch_mfma_w<T, OutT, kD, kKeys, 8>(p, s);
 }
 
