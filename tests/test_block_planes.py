@@ -132,3 +132,52 @@ def test_more_planes_than_one_launch_holds(planes, n_k):
     torch.cuda.synchronize()
     assert torch.equal(out[:-1], one.expand(planes - 1, 1, 16, 32))
     torch.testing.assert_close(out[-1].float(), one[0].float(), rtol=2 ** -8, atol=1e-4)
+
+
+# Many planes: one workgroup per plane (32 dims: 8 and 16 waves, 64 dims: 4, 8
+# and 16, 128 dims: 8 and 16) whose waves take a second and a third query
+# block; without a bias the longer ones are streamed.
+@pytest.mark.parametrize('planes,n_q,n_k,dim', [(1100, 65, 100, 64), (1100, 129, 100, 64), (600, 129, 257, 64),
+                                                (600, 257, 257, 64), (600, 257, 500, 64), (600, 513, 300, 64),
+                                                (300, 250, 600, 64), (600, 129, 300, 32), (600, 257, 1000, 32),
+                                                (1000, 100, 600, 32), (600, 129, 140, 128), (600, 257, 200, 128),
+                                                (1000, 100, 180, 128)])
+@pytest.mark.parametrize('masked', [False, True])
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16], ids=str)
+def test_many_planes_against_float64(planes, n_q, n_k, dim, masked, dtype):
+    print(planes, n_q, n_k, dim, masked, dtype, flush=True)
+    g = torch.Generator(device='cuda').manual_seed(n_q + n_k)
+    q, k, v = (torch.randn(planes, 1, n, dim, generator=g, device='cuda').to(dtype) for n in (n_q, n_k, n_k))
+    scale = torch.full((1, 1, 1, 1), 0.9 / dim, device='cuda')
+    bias = torch.zeros(planes, 1, 1, n_k, device='cuda')
+    if masked:
+        counts = torch.randint(1, n_k + 1, (planes, 1, 1, 1), generator=g, device='cuda')
+        bias.masked_fill_(torch.arange(n_k, device='cuda') >= counts, -math.inf)
+    got = capi.forward(q, k, v, scale, bias if masked else None, out_dtype=torch.float32, variant='tile')
+    for at in (slice(0, 1), slice(planes // 2, planes // 2 + 1), slice(planes - 1, planes)):
+        qd, kd, vd = (t[at, 0].double() for t in (q, k, v))
+        d2 = (qd * qd).sum(-1)[..., None] + (kd * kd).sum(-1)[:, None] - 2 * (qd @ kd.transpose(1, 2).contiguous())
+        want = torch.softmax(bias[at, 0].double() - scale.double().item() * d2, -1) @ vd
+        torch.testing.assert_close(got[at, 0].double(), want, **GATE)
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16], ids=str)
+def test_planes_that_leave_cus_unequal_are_streamed(dtype):
+    """1,000 planes, four workgroups on most CUs: streamed without a bias in 0.6
+    of the time that the workgroups take with one of zeros."""
+    g = torch.Generator(device='cuda').manual_seed(0)
+    q, k, v = (torch.randn(1000, 1, n, 32, generator=g, device='cuda').to(dtype) for n in (100, 1000, 1000))
+    scale = torch.full((1, 1, 1, 1), 0.03, device='cuda')
+    times = {}
+    for name, bias in (('none', None), ('zeros', torch.zeros(1, 1, 1, 1000, device='cuda'))):
+        times[name] = math.inf
+        for _ in range(5):
+            begin, end = torch.cuda.Event(True), torch.cuda.Event(True)
+            begin.record()
+            for _ in range(5):
+                capi.forward(q, k, v, scale, bias, variant='tile')
+            end.record()
+            torch.cuda.synchronize()
+            times[name] = min(times[name], begin.elapsed_time(end))
+    print(times, flush=True)
+    assert times['none'] < 0.8 * times['zeros']

@@ -404,18 +404,60 @@ hipError_t launch_block_k(Problem& p, int64_t splits, int64_t per_split, hipStre
 // 30.1 / 24.9 / 28.1; 1,200 of 130 x 130, 128 dims (83 KB) 94 / 67 / 55; 800 of
 // 400 x 400, 64 dims (108 KB) 134 / 87 / 78; 1,600 of 100 x 100, 64 dims (33 KB)
 // 23.2 / 26.7 / -.  64 planes of 500 x 500 in 512 workgroups 22.3, in 256 14.9.
-template <typename T, typename OutT, int kD>
-hipError_t launch_block_d(Problem& p, hipStream_t s) {
+struct BlockShape {
+  int waves;           // per workgroup
+  int64_t resident;    // workgroups on the chip at once
+  int64_t splits, per;  // workgroups per plane and query blocks of each
+};
+
+template <int kD>
+BlockShape block_shape(const Problem& p) {
+  BlockShape b;
   const int64_t planes = p.B * p.H, blocks = (p.Nq + 15) / 16;
   const int64_t lds = block_lds_bytes<kD>(p.Nk);
-  const int waves = lds <= 40 * 1024 ? 4 : (lds <= 80 * 1024 ? 8 : 16);
-  const int64_t by_lds = kBlockLdsBytes / lds, by_waves = 16 / waves;
-  const int64_t resident = (p.compute_units > 0 ? p.compute_units : 1) * (by_lds < by_waves ? by_lds : by_waves);
-  int64_t splits = resident / planes;
-  if (splits > (blocks + 3) / 4) splits = (blocks + 3) / 4;
-  if (splits < 1) splits = 1;
-  const int64_t per = (blocks + splits - 1) / splits;
-  splits = (blocks + per - 1) / per;
+  b.waves = lds <= 40 * 1024 ? 4 : (lds <= 80 * 1024 ? 8 : 16);
+  const int64_t by_lds = kBlockLdsBytes / lds, by_waves = 16 / b.waves;
+  b.resident = (p.compute_units > 0 ? p.compute_units : 1) * (by_lds < by_waves ? by_lds : by_waves);
+  b.splits = b.resident / planes;
+  if (b.splits > (blocks + 3) / 4) b.splits = (blocks + 3) / 4;
+  if (b.splits < 1) b.splits = 1;
+  b.per = (blocks + b.splits - 1) / b.splits;
+  b.splits = (blocks + b.per - 1) / b.per;
+  return b;
+}
+
+// Whether planes whose keys fit LDS are better streamed by the tile kernel all
+// the same: without a bias, from 256 keys (160 of 128 dims) and two of its
+// items per CU on, by time.  In units of one query block of this kernel on a CU (0.9 us
+// at 600 keys of 64 dims): a workgroup takes its blocks and 7 for the staging,
+// an item of the tile kernel 9.4 (128 rows of 32 dims), 24.6 (256 of 64) or
+// 12.3 (128 of 128), and the fullest CU decides.  Here and streamed, us: 300
+// planes of 700 x 600 x 64 (two workgroups on some CUs, 1.2 on average) 99 and
+// 79, of 700 x 600 x 32 74 and 55, 1000 of 100 x 600 x 32 36 and 31; 256 of
+// 512 x 512 x 64 41 and 43, 128 of 600 x 600 x 64 27 and 42, 256 of
+// 600 x 288 x 128 44 and 55.  fp16 planes of 64 and 128 dims stay: the
+// unshifted weights of rows far from their keys leave fp16's range and take the
+// tile kernel three passes (300 planes of 700 x 350 x 64 65 and 103; at 32 dims
+// rows lie nearer, 1000 of 100 x 1000 x 32 71 and 43).  From 1,024 keys on the
+// tile kernel weighs by fp16: not here.
+template <typename T, int kD>
+bool block_streams(const Problem& p, int64_t most_keys) {
+  if (!__is_same(T, __bf16) && kD != 32) return false;
+  if (p.bias != nullptr || p.Nk < (kD == 128 ? 160 : 256) || p.Nk >= most_keys) return false;
+  const BlockShape b = block_shape<kD>(p);
+  const int64_t planes = p.B * p.H, units = p.compute_units > 0 ? p.compute_units : 1;
+  constexpr int64_t kRows = kD == 64 ? 256 : 128;
+  constexpr double kItem = kD == 32 ? 9.4 : (kD == 64 ? 24.6 : 12.3);
+  const int64_t items = (planes * ((p.Nq + kRows - 1) / kRows) + units - 1) / units;
+  const int64_t staged = (planes * b.splits + units - 1) / units;
+  return items >= 2 && kItem * static_cast<double>(items) < static_cast<double>(staged * (7 + b.per));
+}
+
+template <typename T, typename OutT, int kD>
+hipError_t launch_block_d(Problem& p, hipStream_t s) {
+  const BlockShape b = block_shape<kD>(p);
+  const int waves = b.waves;
+  const int64_t splits = b.splits, per = b.per;
   if (waves == 16) return launch_block_k<T, OutT, kD, 16>(p, splits, per, s);
   if (waves == 8) return launch_block_k<T, OutT, kD, 8>(p, splits, per, s);
   return launch_block_k<T, OutT, kD, 4>(p, splits, per, s);

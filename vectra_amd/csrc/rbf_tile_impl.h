@@ -775,11 +775,15 @@ hipError_t launch_tile_k(Problem& p, hipStream_t s) {
 
 template <typename T, typename OutT>
 hipError_t launch_tile_t(Problem& p, hipStream_t s) {
-  // Planes whose keys fit LDS are staged once for all their queries.
+  // Planes whose keys fit LDS are staged once for all their queries, unless
+  // streaming them is faster (both hold hi + lo weights).
   if (p.Nk <= kBlockMaxKeys) {
-    if (p.D == 32 && block_lds_bytes<32>(p.Nk) <= kBlockLdsBytes) return launch_block_d<T, OutT, 32>(p, s);
-    if (p.D == 64 && block_lds_bytes<64>(p.Nk) <= kBlockLdsBytes) return launch_block_d<T, OutT, 64>(p, s);
-    if (p.D == 128 && block_lds_bytes<128>(p.Nk) <= kBlockLdsBytes) return launch_block_d<T, OutT, 128>(p, s);
+    if (p.D == 32 && block_lds_bytes<32>(p.Nk) <= kBlockLdsBytes && !block_streams<T, 32>(p, kFastKeys))
+      return launch_block_d<T, OutT, 32>(p, s);
+    if (p.D == 64 && block_lds_bytes<64>(p.Nk) <= kBlockLdsBytes && !block_streams<T, 64>(p, kFastKeys))
+      return launch_block_d<T, OutT, 64>(p, s);
+    if (p.D == 128 && block_lds_bytes<128>(p.Nk) <= kBlockLdsBytes && !block_streams<T, 128>(p, kFastKeys))
+      return launch_block_d<T, OutT, 128>(p, s);
   }
   const int64_t planes = p.B * p.H, units = p.compute_units > 0 ? p.compute_units : 1;
   auto items = [&](int64_t cb) { return planes * ((p.Nq + 64 * cb - 1) / (64 * cb)); };
