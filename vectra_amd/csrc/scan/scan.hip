@@ -1412,7 +1412,7 @@ int launch_top_k(int64_t queries, TopK& p, hipStream_t stream) {
 struct FilterPlan {
   TopKFilter f;
   int64_t queries = 0, query_blocks = 0, bytes = 0;  // of a part: the call runs in parts of `queries`
-  int64_t minima = 0, limit = 0, counts = 0, lists = 0;  // byte offsets
+  int64_t minima = 0, limit = 0, centred = 0, centres = 0, counts = 0, lists = 0;  // byte offsets
 };
 
 // The filtered form's four launches take 20-23 us however small the call; the
@@ -1498,6 +1498,8 @@ FilterPlan top_k_filter_part(int64_t queries, const TopK& p) {
   take(kCounterBytes);  // the split form's counters stay as they are
   plan.minima = take(padded * waves * f.group_cols * static_cast<int64_t>(sizeof(float)));
   plan.limit = take(padded * static_cast<int64_t>(sizeof(float)));
+  plan.centred = take(blocks * static_cast<int64_t>(sizeof(uint32_t)));
+  plan.centres = take(blocks * kFilterMaxDim * static_cast<int64_t>(sizeof(float)));
   plan.counts = take(padded * f.workgroups * static_cast<int64_t>(sizeof(uint32_t)));
   plan.lists = take(padded * f.workgroups * kFilterCap * static_cast<int64_t>(sizeof(uint64_t)));
   return plan;
@@ -1544,6 +1546,8 @@ int run_top_k_filter(FilterPlan& plan, int64_t queries, void* workspace, hipStre
   TopKFilter& f = plan.f;
   f.minima = reinterpret_cast<float*>(base + plan.minima);
   f.limit = reinterpret_cast<float*>(base + plan.limit);
+  f.centred = reinterpret_cast<uint32_t*>(base + plan.centred);
+  f.centres = reinterpret_cast<float*>(base + plan.centres);
   f.counts = reinterpret_cast<uint32_t*>(base + plan.counts);
   f.lists = reinterpret_cast<uint64_t*>(base + plan.lists);
   const TopK all = f.t;

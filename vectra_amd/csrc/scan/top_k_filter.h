@@ -8,11 +8,14 @@
 // involved, the reference's distance d lies in
 //
 //   |q|^2 + |r|^2 - 2 q^.r^  -+  (c1 |q||r| + c2 (|q|^2 + |r|^2)),
-//   c1 = 2 (2^-7 + 2^-16 + dim 2^-22),   c2 = (dim + 32) 2^-22
+//   c1 = 2 (2^-7 + 2^-16 + dim 2^-22),   c2 = (dim + 36) 2^-22
 //
 // (Cauchy-Schwarz on the element errors; c2 covers the sums of the norms, of
-// the matrix product and of the reference's own order, with room).  Four
-// launches:
+// the matrix product and of the reference's own order, with room).  Queries
+// that lie together, far from the origin for their spread, are taken from a
+// centre, as are the rows: a shift changes no distance, but the norms above it.
+// The rounding of q - c and r - c moves the distance of the pair by at most
+// 2^-22 (|q - c|^2 + |r - c|^2), which is in c2.  Four launches:
 //
 //  1. top_k_bound_kernel<..., true>: over a sample of the candidates, the
 //     smallest upper end of every group of candidates;
@@ -60,6 +63,8 @@ struct TopKFilter {
   TopK t;
   float* minima;     // [query blocks][groups][64]
   float* limit;      // [query blocks][64]
+  uint32_t* centred;  // [query blocks]: whether the block's queries and the rows are taken from a centre
+  float* centres;     // [query blocks][kFilterMaxDim]
   uint32_t* counts;  // [query blocks][workgroups][64]; above kFilterCap: ran over
   uint64_t* lists;   // [query blocks][workgroups][64][kFilterCap]; of one that ran over, its smallest keys
   int64_t num_queries;
@@ -90,6 +95,14 @@ __device__ __forceinline__ float dpp_min(float x, C) {
 template <typename C>
 __device__ __forceinline__ float dpp_add(float x, C) {
   return x + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), C::value, 0xf, 0xf, false));
+}
+
+// Sums over the four 16-lane rows of a wave, in every lane.
+__device__ __forceinline__ float fold_rows(float x) {
+  auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = __uint_as_float(s[0]) + __uint_as_float(s[1]);
+  s = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(s[0]) + __uint_as_float(s[1]);
 }
 
 // A key in LDS that other waves change meanwhile.
@@ -195,6 +208,7 @@ __global__ __launch_bounds__(kFilterThreads, kSample ? 4 : 3) void top_k_bound_k
   __shared__ __align__(16) float qa[kFilterQueries], qc[kFilterQueries];
   __shared__ float qlimit[kFilterQueries];
   __shared__ uint32_t fill[kFilterQueries];
+  __shared__ __align__(16) float centre[kFilterMaxDim];
   __shared__ uint64_t worst[kSample ? 1 : kFilterQueries];
   __shared__ uint64_t list[kSample ? 1 : kFilterQueries][kSample ? 1 : kFilterCap];
   __shared__ uint32_t queue[kSample ? 1 : kFilterWaves][kSample ? 1 : kFilterQueue];
@@ -213,26 +227,14 @@ __global__ __launch_bounds__(kFilterThreads, kSample ? 4 : 3) void top_k_bound_k
 
   // ---- The block's queries: bf16 fragments, norms, limits.  A thread takes
   // eight dimensions of a query, eight adjacent lanes 64 of them.
-  if (tid < kFilterQueries) qnorm[tid] = 0.f;
-  __syncthreads();
   const bool whole = p.t.query_stride % 4 == 0 && (reinterpret_cast<uintptr_t>(p.t.queries) & 15) == 0;
-#pragma unroll 1
-  for (int item = tid; item < kTiles * 16 * padded * 4; item += kFilterThreads) {
-    const int q = item / (padded * 4);
-    const int d8 = item - q * (padded * 4);  // dimensions 8 d8 .. + 7
-    const float* src = p.t.queries + (q0 + (q < nq ? q : nq - 1)) * p.t.query_stride;
-    float x[8];
-    if (whole && 8 * d8 + 8 <= dim) {
-      const f32x4 lo = *reinterpret_cast<const f32x4*>(src + 8 * d8);
-      const f32x4 hi = *reinterpret_cast<const f32x4*>(src + 8 * d8 + 4);
+  const int items = kTiles * 16 * padded * 4;
+  bool centred = false;
+  // Eight dimensions of a query: its fragment, and its norm's part.
+  auto stage = [&](int q, int d8, float (&x)[8]) {
+    if (centred) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        x[e] = lo[e];
-        x[4 + e] = hi[e];
-      }
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) x[e] = 8 * d8 + e < dim ? src[8 * d8 + e] : 0.f;
+      for (int e = 0; e < 8; ++e) x[e] -= centre[8 * d8 + e];
     }
     bf16x8 f;
     float n = 0.f;
@@ -246,10 +248,99 @@ __global__ __launch_bounds__(kFilterThreads, kSample ? 4 : 3) void top_k_bound_k
     n = dpp_add(n, std::integral_constant<int, 0x4E>{});
     n = dpp_add(n, std::integral_constant<int, 0x141>{});  // row_half_mirror: the other four of eight
     if ((tid & 7) == 0) atomicAdd(&qnorm[q], n);
+  };
+  // The sample finds out whether to take a centre, and the filter is told.
+  if constexpr (!kSample) {
+    centred = p.centred[blockIdx.y] != 0;
+    if (centred && tid < padded * 32) centre[tid] = p.centres[blockIdx.y * kFilterMaxDim + tid];
+  }
+#pragma unroll 1
+  while (true) {
+    if (tid < kFilterQueries) qnorm[tid] = 0.f;
+    __syncthreads();
+    if (whole) {
+      // Loads of four items in flight (all items are whole eights of lanes).
+      constexpr int kAhead = 4;
+#pragma unroll 1
+      for (int first = tid; first < items; first += kAhead * kFilterThreads) {
+        f32x4 part[kAhead][2];
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+          const int item = first + u * kFilterThreads < items ? first + u * kFilterThreads : first;
+          const int q = item / (padded * 4);
+          const int d = 8 * (item - q * (padded * 4));
+          const float* src = p.t.queries + (q0 + (q < nq ? q : nq - 1)) * p.t.query_stride;
+#pragma unroll
+          for (int h = 0; h < 2; ++h) part[u][h] = *reinterpret_cast<const f32x4*>(src + (d + 4 * h < dim ? d + 4 * h : 0));
+        }
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+          const int item = first + u * kFilterThreads;
+          if (item >= items) break;
+          const int q = item / (padded * 4);
+          const int d8 = item - q * (padded * 4);
+          float x[8];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) x[e] = 8 * d8 + (e & 4) < dim ? part[u][e / 4][e % 4] : 0.f;
+          stage(q, d8, x);
+        }
+      }
+    } else {
+#pragma unroll 1
+      for (int item = tid; item < items; item += kFilterThreads) {
+        const int q = item / (padded * 4);
+        const int d8 = item - q * (padded * 4);  // dimensions 8 d8 .. + 7
+        const float* src = p.t.queries + (q0 + (q < nq ? q : nq - 1)) * p.t.query_stride;
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = 8 * d8 + e < dim ? src[8 * d8 + e] : 0.f;
+        stage(q, d8, x);
+      }
+    }
+    __syncthreads();
+    if (!kSample || centred) break;
+    // The first m (at most 16) queries lie together where their mean's square
+    // is over three quarters of the mean of their squares (a shift of 1.7
+    // deviations an element): the sum of their products with each other
+    // against that of their squares.  A NaN is not over it.  Every workgroup of
+    // the query block computes the same bits.  256 queries x 50,000 x 96, k = 10,
+    // bounded from the origin and from the centre, us (exact search 540): no
+    // shift 54 and 61, 2 deviations 63 and 62, 4 272 and 62, 8 1,193 and 61.
+    const int m = nq < 16 ? nq : 16;
+    f32x4 gram = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int c = 0; c < padded; ++c)
+      gram = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qfrag[c * kWaveLanes + lane], qfrag[c * kWaveLanes + lane], gram, 0, 0, 0);
+    float over = 0.f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = 4 * grp + r;
+      const float g = row == col ? gram[r] * (1.f - 0.75f * static_cast<float>(m)) : gram[r];
+      over += row < m && col < m ? g : 0.f;
+    }
+    over = dpp_add(over, std::integral_constant<int, 0xB1>{});
+    over = dpp_add(over, std::integral_constant<int, 0x4E>{});
+    over = dpp_add(over, std::integral_constant<int, 0x141>{});
+    over = dpp_add(over, std::integral_constant<int, 0x140>{});  // row_mirror
+    over = fold_rows(over);
+    centred = __builtin_amdgcn_readfirstlane(over > 0.f) != 0;
+    if (!centred) break;
+    if (tid < padded * 32) {
+      float sum = 0.f;
+      if (tid < dim)
+        for (int q = 0; q < m; ++q) sum += p.t.queries[(q0 + q) * p.t.query_stride + tid];
+      centre[tid] = sum / static_cast<float>(m);
+    }
+    // (The loop's first barrier lies between the centre and its use, and
+    // between the products above and the new fragments.)
+  }
+  if constexpr (kSample) {
+    if (blockIdx.x == 0) {
+      if (tid == 0) p.centred[blockIdx.y] = centred ? 1u : 0u;
+      if (centred && tid < padded * 32) p.centres[blockIdx.y * kFilterMaxDim + tid] = centre[tid];
+    }
   }
   const float c1 = 2.f * (0x1p-7f + 0x1p-16f + static_cast<float>(dim) * 0x1p-22f);
-  const float c2 = static_cast<float>(dim + 32) * 0x1p-22f;
-  __syncthreads();
+  const float c2 = static_cast<float>(dim + 36) * 0x1p-22f;
   if (tid < kFilterQueries) {
     const float n = qnorm[tid], length = sqrtf(n);
     if constexpr (kSample) {
@@ -377,13 +468,7 @@ __global__ __launch_bounds__(kFilterThreads, kSample ? 4 : 3) void top_k_bound_k
   // The bounds of a tile whose products are complete.
   auto finish = [&](int i, bool ok) {
     // |r|^2 of the lane's candidate: its four lane groups hold a part each.
-    float rn = norm;
-    {
-      auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(rn), __float_as_uint(rn), false, false);
-      rn = __uint_as_float(s[0]) + __uint_as_float(s[1]);
-      s = __builtin_amdgcn_permlane32_swap(__float_as_uint(rn), __float_as_uint(rn), false, false);
-      rn = __uint_as_float(s[0]) + __uint_as_float(s[1]);
-    }
+    const float rn = fold_rows(norm);
     const float length = sqrtf(rn);
     if constexpr (kSample) {
       const float rb = rn * (1.f + c2);
@@ -460,8 +545,10 @@ __global__ __launch_bounds__(kFilterThreads, kSample ? 4 : 3) void top_k_bound_k
         bf16x8 f;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
+          const int d = (slab * kChunks + c) * 32 + 8 * grp + 4 * h;
           f32x4 v = x[c][h];
-          if (partial && (slab * kChunks + c) * 32 + 8 * grp + 4 * h >= dim) v = f32x4{0.f, 0.f, 0.f, 0.f};
+          if (centred) v -= *reinterpret_cast<const f32x4*>(&centre[d]);
+          if (partial && d >= dim) v = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             f[4 * h + e] = static_cast<__bf16>(v[e]);
