@@ -425,11 +425,12 @@ __device__ __forceinline__ float adc_sum_words(const uint4 (&chunk)[kChunks], in
   return sum;
 }
 
-// Workgroups of the 16-byte ADC scan: 512 threads, four per compute unit
-// (kAdcBlocks over the 256 CUs of an MI355X), so the table is staged 1024
+constexpr int64_t kComputeUnits = 256;  // of an MI355X, the one target
+
+// Workgroups of the 16-byte ADC scan: 512 threads, four per compute unit, so the table is staged 1024
 // times per launch instead of once per 256 codes.
 constexpr int kAdcThreads = 512;
-constexpr int64_t kAdcBlocks = 1024;
+constexpr int64_t kAdcBlocks = 4 * kComputeUnits;
 
 // Each lane sums one code per step and holds two steps' codes in two register
 // sets: the next step's code is requested before the current one is summed.
@@ -1209,7 +1210,7 @@ int launch_adc_multi_k(PqAdc& p, int64_t queries, hipStream_t stream) {
   const int64_t y = (queries + kQ - 1) / kQ;
   const size_t lds = static_cast<size_t>(p.subspaces) * VECTRA_PQ_CENTROIDS * kQ * sizeof(float);
   const int64_t per_cu = lds <= 80 * 1024 ? 2 : 1;
-  int64_t x = (256 * per_cu + y - 1) / y;
+  int64_t x = (kComputeUnits * per_cu + y - 1) / y;
   const dim3 grid(blocks_for(p.num_cand, kAdcMultiThreads, x < 1 ? 1 : x), static_cast<unsigned>(y));
   const void* kernel = p.ids != nullptr ? reinterpret_cast<const void*>(&pq_adc_multi_kernel<kQ, kWords, kM, true>)
                                         : reinterpret_cast<const void*>(&pq_adc_multi_kernel<kQ, kWords, kM, false>);
@@ -1470,7 +1471,8 @@ FilterPlan top_k_filter_part(int64_t queries, const TopK& p) {
   }
   if (waves * f.group_cols < 3 * p.k || waves * f.group_cols > kFilterMaxGroups) return plan;
   f.sample_waves = static_cast<int32_t>(waves);
-  // A quarter of the candidates; half where many results are wanted, whose
+  // A quarter of the candidates, rounded up to whole tiles for every wave (a
+  // third of 200,000 for 64 queries); half where many results are wanted, whose
   // surviving pairs then cost more than the sample does (1,024 queries, 12,500
   // rows, k = 100: 121 us with a quarter, 87 with half; 8 queries, 500,000
   // rows: 49 and 53).
@@ -1478,10 +1480,11 @@ FilterPlan top_k_filter_part(int64_t queries, const TopK& p) {
   const int64_t each = (f.tiles / share + waves - 1) / waves;
   f.sample_tiles = static_cast<int32_t>(each < 1 ? 1 : (each * waves > f.tiles ? f.tiles / waves : each));
   f.sample_step = static_cast<int32_t>(f.tiles / (waves * f.sample_tiles));
-  // The filter: up to 768 workgroups (three per CU, all resident at once), at
-  // least one per two results, so that a workgroup's share of the k nearest
-  // is a few.
-  int64_t wgs = 768 / blocks;
+  // The filter: as many workgroups as are resident at once (three per CU; two
+  // where the fragments of 64 queries of more than 128 dimensions take 32 KB of
+  // LDS beside the 28 KB of queues and lists), at least one per two results, so
+  // that a workgroup's share of the k nearest is a few.
+  int64_t wgs = kComputeUnits * (p.dim > 128 && queries > 16 ? 2 : 3) / blocks;
   if (wgs < p.k / 2) wgs = p.k / 2;
   if (wgs < 1) wgs = 1;
   const int64_t per_wave = (f.tiles + wgs * kFilterWaves - 1) / (wgs * kFilterWaves);
