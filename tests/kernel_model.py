@@ -22,7 +22,13 @@ unless the weight sums leave the range where the split is accurate
 16 queries of a block together and recomputes the whole block with each
 query's own maximum logit subtracted; the tile kernel takes the exact passes
 (a maximum pass, then a shifted pass) for every query of its work item when
-a bias is present, gamma < 0, or any sum falls below the range.
+gamma < 0 or any sum falls below the range.
+
+With a bias the model shifts by each query's own maximum.  The kernels (the tile
+kernel, and those that stage a plane whole or share its keys out) shift by its
+largest logit over a part of the keys and take the exact maximum only where the
+sum then leaves the range: the same weights up to one common factor inside it,
+so within the split's 2^-17 of the model.
 
 The tile kernel's fast pass (no bias, gamma >= 0, at least FAST_KEYS keys)
 comes first: each weight rounded once to fp16 (to nearest), no split, and the

@@ -1,5 +1,5 @@
 """16-bit planes beyond one tile with a key bias or query counts that split
-unevenly: planes staged whole in LDS (up to 160 KB: 310 to 1,024 keys by head
+unevenly: planes staged whole in LDS (up to 160 KB: 288 to 1,024 keys by head
 width) and streamed key tiles, at the sizes where the staging, the key pairs,
 the waves and the work items end (GPU, through the C ABI)."""
 
@@ -35,8 +35,8 @@ def _run(q, k, v, scale, bias, variant='tile'):
     return got.cpu().double()
 
 
-# 64 dims: 630 keys fit (4 waves up to 157, 8 up to 314, 16 above); 32 dims:
-# all up to 1,024; 128 dims: 317.  Longer planes stream.
+# Keys are staged in pairs of 16.  64 dims: 608 keys fit (4 waves up to 128, 8 up
+# to 288, 16 above); 32 dims: all up to 1,024; 128 dims: 288.  Longer planes stream.
 @pytest.mark.parametrize('n_q,n_k,dim', [(16, 1, 64), (17, 31, 64), (33, 32, 64), (81, 33, 64), (100, 150, 64),
                                          (257, 257, 64), (65, 315, 64), (20, 608, 64), (130, 641, 64), (300, 1023, 64),
                                          (18, 81, 32), (129, 300, 32), (260, 1000, 32), (40, 1024, 32), (70, 1030, 32),

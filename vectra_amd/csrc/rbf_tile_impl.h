@@ -25,7 +25,7 @@
 // Without a bias and with gamma >= 0, x <= 0 (d >= 0 up to rounding), so
 // exp2(x) is used as the weight directly: one pass over the keys, no running
 // maximum and no rescaling.  With a bias, one pass too: each query's weights
-// are shifted by its largest logit over the first tile.  If a query's weight
+// are shifted by its largest logit over the first tile with a key that counts.  If a query's weight
 // sum then ends outside the range in which the 16-bit split is accurate (the
 // query is far from every key, later keys weigh far more than the first), and
 // always for gamma < 0 without a bias, the item is computed exactly: one pass
@@ -146,7 +146,9 @@ constexpr float kFastWalk = kFastSigmas * 0x1p-11f * 0.57735026919f;  // kFastSi
 // for 32-dim heads; four blocks at two waves per SIMD for 64-dim heads (each
 // K and V^T fragment, and each tile's staging, then serve 64 queries per
 // wave: 10 % faster at config 4 than two blocks at three waves); 128-dim
-// heads keep two blocks at two waves.
+// heads keep two blocks at two waves.  Spilled vector registers, bf16: four
+// blocks of 64 dims 15 (18 with a bias), two with a bias 15, the rest none
+// (128 dims with a bias: 245 of 256 registers).
 template <typename T, typename OutT, int kD, int kKeys, int kWaves, int kCB, bool kBias>
 __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kD <= 64 && kCB <= 2 ? 3 : 2))) void
 rbf_tile_kernel(Problem p, int32_t q_blocks) {
