@@ -51,7 +51,8 @@ def _long_axis(n_q, n_k, dim):
     return [t.bfloat16() for t in (q, k, v)] + [torch.full((1, 1, 1, 1), 0.64 / dim, device='cuda')]
 
 
-@pytest.mark.parametrize('n_q,n_k,dim', [(600, 2048, 64), (64, 1025, 64), (257, 1601, 64), (300, 2048, 32), (129, 1100, 32),
+@pytest.mark.parametrize('n_q,n_k,dim', [(600, 2048, 64), (64, 1025, 64), (257, 1601, 64), (100, 1200, 64),
+                                         (128, 1100, 64), (65, 1100, 64), (60, 1100, 32), (300, 2048, 32), (129, 1100, 32),
                                          (200, 1100, 128)])
 @pytest.mark.parametrize('out_dtype', [torch.float32, torch.bfloat16], ids=str)
 def test_rows_do_not_depend_on_the_planes_beside_them(n_q, n_k, dim, out_dtype):

@@ -801,10 +801,22 @@ hipError_t launch_tile_t(Problem& p, hipStream_t s) {
   // blocks and 132 with one where the fp16 pass holds, 251 and 218 where it does
   // not; 32 of 3000 x 3000 126 and 113, 265 and 207.  (Smaller items whose
   // groups agree through two further launches: 135 and 256, 117 and 231.)
+  // The same rows may be cut otherwise: a plane of at most 64 or 128 rows is one
+  // item of fewer blocks, and where a CU has one item at most, eight waves of
+  // half the blocks hide more of its latency.  Four blocks and these, us: 200
+  // planes of 62 x 2892 x 64 188 and 103, 40 of 119 x 3136 x 64 188 and 103, 8 of
+  // 700 x 3000 x 64 182 and 146, 64 of 1000 x 4096 x 64 261 and 227.
   if (p.bias == nullptr) {
     switch (p.D) {
-      case 32: return launch_tile_k<T, OutT, 32, 64, 4, 2, false>(p, s);
-      case 64: return launch_tile_k<T, OutT, 64, 64, 4, 4, false>(p, s);
+      case 32:
+        if (p.Nq <= 64) return launch_tile_k<T, OutT, 32, 64, 4, 1, false>(p, s);
+        return launch_tile_k<T, OutT, 32, 64, 4, 2, false>(p, s);
+      case 64:
+        if (p.Nq <= 64) return launch_tile_k<T, OutT, 64, 64, 4, 1, false>(p, s);
+        if (p.Nq <= 128 && planes <= units) return launch_tile_k<T, OutT, 64, 64, 8, 1, false>(p, s);
+        if (p.Nq <= 128) return launch_tile_k<T, OutT, 64, 64, 4, 2, false>(p, s);
+        if (items(4) <= units) return launch_tile_k<T, OutT, 64, 64, 8, 2, false>(p, s);
+        return launch_tile_k<T, OutT, 64, 64, 4, 4, false>(p, s);
       case 128: return launch_tile_k<T, OutT, 128, 32, 4, 2, false>(p, s);
       default: return hipErrorInvalidValue;
     }
